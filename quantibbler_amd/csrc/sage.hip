@@ -122,7 +122,29 @@ struct RefArgs {
     int *gpv;         // [dv][rows]
     float *gout;      // [dv][rows]
     int sc_lds, out_lds;
+    // > 0: khat and vhat in sage_ref_tile's fragment order (ref_k_word,
+    // ref_v_word) for this many keys a lane, nv 16-channel tiles of V
+    uint32_t kpl, nv;
 };
+
+// Where sage_ref_tile's operands keep a code word of key block (bk, kb): a
+// fragment is the 64 lanes' 16 bytes (V's of short blocks: 4 kpl / 4) in a
+// row, so that a wave loads it with consecutive lanes on consecutive bytes
+// (gathered from row-major codes the kernel took 124 us a call against 117).
+// K^ word w4 (channels 4 w4 ..) of the block's key kk: A row (kk / kpl,
+// kk % 4) of 16-key tile (kk % kpl) / 4.
+__device__ __forceinline__ size_t ref_k_word(const RefArgs &a, size_t bk, size_t kb, uint32_t kk, uint32_t w4) {
+    const uint32_t nt = a.kpl / 4, dk = (uint32_t)a.d4 / 16;
+    const uint32_t kt = kk % a.kpl / 4, row = 4 * (kk / a.kpl) + kk % 4;
+    const uint32_t lane = 16 * (w4 % 16 / 4) + row;
+    return (((bk * a.pnkb + kb) * nt + kt) * dk + w4 / 16) * 256 + lane * 4 + w4 % 4;
+}
+// V^ word w4 (keys 4 w4 ..) of channel c: lane (c % 16, the keys' group)
+__device__ __forceinline__ size_t ref_v_word(const RefArgs &a, size_t bk, size_t kb, uint32_t c, uint32_t w4) {
+    const uint32_t wpl = a.kpl / 4, nj = wpl > 4 ? wpl / 4 : 1, fw = wpl < 4 ? wpl : 4;
+    const uint32_t r = w4 % wpl, lane = 16 * (w4 / wpl) + c % 16;
+    return (((bk * a.pnkb + kb) * a.nv + c / 16) * nj + r / 4) * (64 * fw) + lane * fw + r % 4;
+}
 
 // Pre-pass: one workgroup per (kv head, key block).  gpu_attention.rs:192-204
 // (block mean, sequential over the block's tokens), :211-226 (per-token peak
@@ -150,6 +172,8 @@ __global__ void __launch_bounds__(256) sage_ref_prep(RefArgs a) {
     const float *V = a.v + bk * a.v_head;
     const size_t maxd = a.d > a.dv ? a.d : a.dv, CH = ref_prep_ch(maxd);
     const bool one = kj <= CH;  // the whole block in one chunk: load once
+    // with two grid layers K and V have a workgroup each, else one does both
+    const bool do_k = gridDim.z == 1 || blockIdx.z == 0, do_v = gridDim.z == 1 || blockIdx.z == 1;
     const int tid = threadIdx.x, nt = blockDim.x;
     const int lane = tid & 63, wave = tid >> 6, nwave = nt >> 6;
     // tokens t0 .. t0+tc-1 (w channels each) into the tile: a wave per token,
@@ -192,17 +216,20 @@ __global__ void __launch_bounds__(256) sage_ref_prep(RefArgs a) {
                       kj * vq <= 8 * (size_t)nt;
     const uint32_t nkq = (uint32_t)kj * dq, nvq = (uint32_t)kj * vq;
     f32x4_t vr[8];
+    if (fast && do_v) {
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const uint32_t it = (uint32_t)(tid + u * nt), i = it < nvq ? it : nvq - 1;
+            vr[u] = *(const f32x4_t *)(V + (j0 + i / vq) * a.v_tok + 4 * (i % vq));
+        }
+    }
+    if (do_k) {
     if (fast) {
         f32x4_t kr[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             const uint32_t it = (uint32_t)(tid + u * nt), i = it < nkq ? it : nkq - 1;
             kr[u] = *(const f32x4_t *)(K + (j0 + i / dq) * a.k_tok + 4 * (i % dq));
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const uint32_t it = (uint32_t)(tid + u * nt), i = it < nvq ? it : nvq - 1;
-            vr[u] = *(const f32x4_t *)(V + (j0 + i / vq) * a.v_tok + 4 * (i % vq));
         }
 #pragma unroll
         for (int u = 0; u < 8; u++) {
@@ -257,10 +284,14 @@ __global__ void __launch_bounds__(256) sage_ref_prep(RefArgs a) {
             if ((size_t)wl < a.d4) {
                 int c4[4];
                 for (int e = 0; e < 4; e++) c4[e] = c0 + e < a.d ? q8(g[e] / kdelta) : 0;
-                a.khat[(bk * a.pst + jj) * a.d4 + wl] = pack4(c4[0], c4[1], c4[2], c4[3]);
+                const size_t at = a.kpl ? ref_k_word(a, bk, kb, (uint32_t)(jj - j0), (uint32_t)wl)
+                                        : (bk * a.pst + jj) * a.d4 + wl;
+                a.khat[at] = pack4(c4[0], c4[1], c4[2], c4[3]);
             }
         }
     }
+    }
+    if (!do_v) return;
     // V: per-channel peak over the block, then codes four tokens a word
     float vpeak = 0.0f;
     for (size_t t0 = j0; t0 < j1; t0 += CH) {
@@ -305,7 +336,11 @@ __global__ void __launch_bounds__(256) sage_ref_prep(RefArgs a) {
                 const size_t t = 4 * w + e;
                 c4[e] = t < tc ? q8(tile[t * maxd + c] / vd) : 0;
             }
-            vrow[c * a.blk4 + (t0 - j0) / 4 + w] = pack4(c4[0], c4[1], c4[2], c4[3]);
+            const uint32_t word = pack4(c4[0], c4[1], c4[2], c4[3]);
+            if (a.kpl)
+                a.vhat[ref_v_word(a, bk, kb, c, (uint32_t)((t0 - j0) / 4) + w)] = word;
+            else
+                vrow[c * a.blk4 + (t0 - j0) / 4 + w] = word;
         }
     }
 }
@@ -490,6 +525,396 @@ __global__ void __launch_bounds__(REF_ROWS) sage_ref_main(RefArgs a) {
         for (size_t c = 0; c < dv; c++) a.out[row * dv + c] = OUT(c) / ell;
 }
 
+// ---- main pass on the matrix cores -----------------------------------------
+//
+// sage_ref_main's arithmetic for key blocks of at most 128 tokens and head
+// dims of at most 128: both INT8 products on v_mfma_i32_16x16x64_i8 (exact
+// integers, so any order gives sage_ref_main's values) and the f32 sequence
+// unchanged, element by element.
+//
+// What bounds it: the VALU work of the softmax, ~50 operations a score (the
+// exp's unfused polynomial alone is 24) -- so the split gives every lane of
+// a wave scores to work on.  A wave owns 16 queries (four waves a workgroup:
+// 64 consecutive queries of one head), S^T = K^ Q^^T with the keys as MFMA
+// rows: lane (col, G) holds query col's scores of the KPL consecutive keys
+// KPL G .. KPL G + KPL - 1 of the block (the row a lane of the A operand
+// loads is chosen so), which is the B operand layout of the second product
+// O^T += V^^T P^^T as well: the codes of P never leave their lane.  Only the
+// sums the reference orders cross lanes:
+//  * sum p of a block in key order: the four lane groups add their keys in
+//    turn, the running sum handed from one to the next;
+//  * the shift sum_c (q^_c dq) kmean_c in channel order: a lane per query,
+//    each wave one of the next four key blocks (products q^ dq in LDS, the
+//    block's means loaded a group ahead), four blocks at a time.
+// A wave's dependent chain per key block (softmax ~2200 cycles, the output
+// update ~1000, the shifts ~500; few waves a SIMD) sets the pace: K^ and its
+// deltas are loaded a block ahead and V^ ahead of the softmax, so that no
+// load is waited for.  Measured (16 / 8 heads, d 128, 1999 tokens, causal,
+// block 64): a query per lane and v_dot4 (sage_ref_main) 10.16 ms a call,
+// this 0.109 ms; block 128 at 1800 tokens, 8 heads, 9.05 -> 0.095 ms; d 64,
+// block 32, not causal, 1900 tokens, 8 heads, 5.18 -> 0.085 ms.
+#define REF_TILE_Q 64  // queries a workgroup
+#define REF_TILE_AHEAD 4  // key blocks whose shifts are formed together (one a wave)
+
+// qbk_expf for x <= 0 or NaN, the same value bit for bit (compared over
+// every float of that range on gfx950): p 2^n by v_ldexp_f32, which rounds
+// once into the subnormals as the two exponent-field products do.
+__device__ __forceinline__ float qbk_expf_neg(float x) {
+    const float log2e = 1.44269504088896341f;
+    const float ln2_hi = 0.693145751953125f;
+    const float ln2_lo = 1.428606765330187045e-06f;
+    const float n = __builtin_rintf(x * log2e);
+    float r = x - n * ln2_hi;
+    r = r - n * ln2_lo;
+    float p = 1.0f / 5040.0f;
+    p = p * r + 1.0f / 720.0f;
+    p = p * r + 1.0f / 120.0f;
+    p = p * r + 1.0f / 24.0f;
+    p = p * r + 1.0f / 6.0f;
+    p = p * r + 0.5f;
+    p = p * r + 1.0f;
+    p = p * r + 1.0f;
+    p = __builtin_amdgcn_ldexpf(p, (int)n);
+    return x < -103.97208f ? 0.0f : p;
+}
+
+typedef int ref_i32x4_t __attribute__((ext_vector_type(4)));
+// 4-byte aligned vectors: rows of the pre-pass products start at any word
+typedef float ref_f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
+
+// the largest of the four lanes l, l ^ 16, l ^ 32, l ^ 48 (NaN loses, as in
+// the reference's `>`)
+__device__ __forceinline__ float ref_max4(float v) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    const float m = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+// The sum over lane groups G = 0 .. 3 in order of their p[0 .. n), from
+// +0.0: group G continues from group G - 1's running sum.  permlane16_swap
+// of a register with itself gives row 1 row 0's value (and row 3 row 2's),
+// its other result rows 0 and 2 those of rows 1 and 3; permlane32_swap the
+// same with the halves of the wave.
+template <int N>
+__device__ __forceinline__ float ref_ordered_sum(const float *p) {
+    auto add = [&](float c) {
+#pragma unroll
+        for (int e = 0; e < N; e++) c += p[e];
+        return c;
+    };
+    auto lo16 = [](float v) {  // rows 0, 0, 2, 2
+        return __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false)[0]);
+    };
+    auto hi16 = [](float v) {  // rows 1, 1, 3, 3
+        return __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false)[1]);
+    };
+    auto lo32 = [](float v) {  // the lower half in both
+        return __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false)[0]);
+    };
+    auto hi32 = [](float v) {
+        return __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false)[1]);
+    };
+    float c = add(0.0f);        // right in row 0
+    c = add(lo16(c));           // right in row 1
+    c = add(lo32(hi16(c)));     // right in row 2
+    c = add(lo16(c));           // right in row 3
+    return hi32(hi16(c));
+}
+
+// KPL: keys a lane holds of a block (the block's keys over four lane groups,
+// 4, 8, 16 or 32); DK: 64-channel steps of the head dim; NV: 16-channel
+// tiles of the value dim.
+template <int KPL, int DK, int NV>
+__global__ void __launch_bounds__(256, KPL == 32 ? 1 : 2) sage_ref_tile(RefArgs a, uint32_t hpx) {
+    constexpr int NT = KPL / 4;                    // 16-key MFMA tiles of a block
+    constexpr int NJ = KPL > 16 ? KPL / 16 : 1;    // 64-key steps of the second product
+    __shared__ __attribute__((aligned(16))) float qdl[16 * DK * REF_TILE_Q * 4];  // q^ dq [c / 4][query][c % 4]
+    __shared__ float shl[REF_TILE_AHEAD][REF_TILE_Q];
+    __shared__ __attribute__((aligned(16))) float kml[REF_TILE_AHEAD][64 * DK];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, G = lane >> 4;
+    const uint32_t nq = (uint32_t)((a.S + REF_TILE_Q - 1) / REF_TILE_Q), BH = (uint32_t)(a.B * a.H);
+    // longest key ranges first; workgroup i runs on XCD i mod 8, which then
+    // keeps to hpx heads (their codes stay in its L2)
+    const uint32_t L = blockIdx.x;
+    uint32_t bh, qi;
+    {
+        const uint32_t nh = hpx ? hpx : BH;
+        const uint32_t s = hpx ? L / 8 : L;
+        bh = (hpx ? (L % 8) * hpx : 0) + s % nh;
+        qi = nq - 1 - s / nh;
+    }
+    const size_t b = bh / a.H, h = bh % a.H;
+    const size_t bk = b * a.Hk + h / (a.H / a.Hk);
+    const uint32_t S = (uint32_t)a.S, blk = (uint32_t)(a.block < a.S ? a.block : a.S);
+    const uint32_t d = (uint32_t)a.d, dv = (uint32_t)a.dv;
+    const uint32_t q0 = qi * REF_TILE_Q, qw = q0 + 16 * wave;
+    const uint32_t i = qw + col;              // this lane's query
+    const uint32_t iq = i < S ? i : S - 1;    // past the last: it repeats the last one's and stores nothing
+
+    // psi_Q (gpu_attention.rs:113-159): lane (col, G) forms channels
+    // 64 dc + 16 G .. + 15 of its query, the B operand's layout
+    float qdelta = 1.0f;
+    ref_i32x4_t qf[DK];
+    {
+        const float *qr = a.q + ((size_t)bh * a.S + iq) * a.d;
+        float x[DK][16];
+        float pk = 0.0f;
+#pragma unroll
+        for (int dc = 0; dc < DK; dc++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) {  // clamped, so that every load is issued at once
+                const uint32_t c = 64 * dc + 16 * G + e;
+                x[dc][e] = qr[c < d ? c : d - 1];
+            }
+#pragma unroll
+        for (int dc = 0; dc < DK; dc++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) {
+                const uint32_t c = 64 * dc + 16 * G + e;
+                x[dc][e] = c < d ? x[dc][e] * a.inv_sqrt_d : 0.0f;
+                pk = fmaxf(pk, fabsf(x[dc][e]));
+            }
+        pk = ref_max4(pk);
+        if (pk > 0.0f) qdelta = pk / 127.0f;
+#pragma unroll
+        for (int dc = 0; dc < DK; dc++)
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+                int c4[4];
+                f32x4_t pr;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    c4[e] = q8(x[dc][4 * w + e] / qdelta);
+                    pr[e] = (float)c4[e] * qdelta;
+                }
+                qf[dc][w] = (int)pack4(c4[0], c4[1], c4[2], c4[3]);
+                *(f32x4_t *)&qdl[((16 * dc + 4 * G + w) * REF_TILE_Q + 16 * wave + col) * 4] = pr;
+            }
+    }
+
+    // key blocks of this lane's query, of the wave's queries, of the workgroup's
+    const uint32_t nkb = (uint32_t)a.nkb;
+    const uint32_t ql = q0 + REF_TILE_Q - 1 < S ? q0 + REF_TILE_Q - 1 : S - 1;
+    const uint32_t wl = qw + 15 < S ? qw + 15 : S - 1;
+    const uint32_t kb_wg = a.causal ? ql / blk + 1 : nkb;
+    const uint32_t kb_wave = qw >= S ? 0 : a.causal ? wl / blk + 1 : nkb;
+    const uint32_t kb_first = a.causal ? qw / blk + 1 : nkb;  // the wave's first query's (the fewest)
+    const uint32_t kb_lane = a.causal ? iq / blk + 1 : nkb;
+
+    f32x4_t o[NV];
+#pragma unroll
+    for (int ct = 0; ct < NV; ct++) o[ct] = f32x4_t{0, 0, 0, 0};
+    float m = MASKED, ell = 0.0f;
+    // key block kb's codes (A operand: tile kt's row `col` is key KPL (col /
+    // 4) + 4 kt + col % 4) and deltas, loaded a block ahead; keys past the
+    // block read whatever is there and whatever follows its deltas (within
+    // the workspace): their scores are masked
+    ref_i32x4_t kf[NT][DK];
+    ref_f32x4u_t kd[NT];
+    auto load_k = [&](uint32_t kb) {
+        const ref_i32x4_t *kh = (const ref_i32x4_t *)a.khat + (bk * a.pnkb + kb) * (NT * DK * 64) + lane;
+        const float *kdp = a.kdelta + bk * a.pst + kb * blk + KPL * G;
+#pragma unroll
+        for (int kt = 0; kt < NT; kt++) {
+#pragma unroll
+            for (int dc = 0; dc < DK; dc++) kf[kt][dc] = kh[(kt * DK + dc) * 64];
+            kd[kt] = *(const ref_f32x4u_t *)(kdp + 4 * kt);
+        }
+    };
+    float kmr[DK];
+    auto load_km = [&](uint32_t kb) {
+        const float *km = a.kmean + (bk * a.pnkb + (kb < kb_wg ? kb : kb_wg - 1)) * a.d;
+#pragma unroll
+        for (int u = 0; u < DK; u++) kmr[u] = km[(uint32_t)(64 * u + lane) < d ? 64 * u + lane : 0];
+    };
+    load_km(wave);
+    if (kb_wave) load_k(0);
+    for (uint32_t kb = 0; kb < kb_wg; kb++) {
+        if (kb % REF_TILE_AHEAD == 0) {  // the shifts of key blocks kb .. kb + 3 (:253), one a wave
+            __syncthreads();
+            if (kb + wave < kb_wg) {
+                // the wave's block's means, loaded a group ago, through LDS
+                // (a wave's LDS accesses complete in order)
+#pragma unroll
+                for (int u = 0; u < DK; u++) kml[wave][64 * u + lane] = kmr[u];
+                load_km(kb + REF_TILE_AHEAD + wave);
+                const float *km = kml[wave];
+                float sh = 0.0f;
+                uint32_t c = 0;
+                for (; c + 32 <= d; c += 32) {
+                    f32x4_t pr[8], kq[8];
+#pragma unroll
+                    for (int w = 0; w < 8; w++) {
+                        pr[w] = *(const f32x4_t *)&qdl[((c / 4 + w) * REF_TILE_Q + lane) * 4];
+                        kq[w] = *(const f32x4_t *)&km[c + 4 * w];
+                    }
+#pragma unroll
+                    for (int e = 0; e < 32; e++) sh += pr[e / 4][e % 4] * kq[e / 4][e % 4];
+                }
+                for (; c < d; c++) sh += qdl[((c / 4) * REF_TILE_Q + lane) * 4 + c % 4] * km[c];
+                shl[wave][lane] = sh;
+            }
+            __syncthreads();
+        }
+        if (kb >= kb_wave) continue;
+        const uint32_t j0 = kb * blk, kj = S - j0 < blk ? S - j0 : blk;
+        // scores (:209-262)
+        const float shift = shl[kb % REF_TILE_AHEAD][16 * wave + col];
+        float p[KPL];
+#pragma unroll
+        for (int kt = 0; kt < NT; kt++) {
+            ref_i32x4_t acc = {0, 0, 0, 0};
+#pragma unroll
+            for (int dc = 0; dc < DK; dc++)
+                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf[kt][dc], qf[dc], acc, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; e++) p[4 * kt + e] = (float)acc[e] * qdelta * kd[kt][e] + shift;
+        }
+        // this block's V^^T fragments (channel 16 ct + col, this lane group's
+        // keys) and deltas (channels past dv read another block's, within the
+        // workspace, and are not stored), then the next block's K^
+        ref_i32x4_t vf[NJ][NV];
+        ref_f32x4u_t dl[NV];
+        {
+            constexpr int FW = KPL < 16 ? KPL / 4 : 4;  // words of a lane in a fragment
+            const uint32_t *vh = a.vhat + ((bk * a.pnkb + kb) * (NV * NJ * 64) + lane) * FW;
+            const float *vd = a.vd + (bk * a.pnkb + kb) * a.dv + 4 * G;
+#pragma unroll
+            for (int ct = 0; ct < NV; ct++) {
+#pragma unroll
+                for (int j = 0; j < NJ; j++) {
+                    const uint32_t *vr = vh + (ct * NJ + j) * (64 * FW);
+                    if constexpr (KPL >= 16) {
+                        vf[j][ct] = *(const ref_i32x4_t *)vr;
+                    } else if constexpr (KPL == 8) {
+                        const uint2 w = *(const uint2 *)vr;
+                        vf[j][ct] = ref_i32x4_t{(int)w.x, (int)w.y, 0, 0};
+                    } else {
+                        vf[j][ct] = ref_i32x4_t{(int)vr[0], 0, 0, 0};
+                    }
+                }
+                dl[ct] = *(const ref_f32x4u_t *)(vd + 16 * ct);
+            }
+        }
+        load_k(kb + 1 < kb_wave ? kb + 1 : kb);
+        __builtin_amdgcn_sched_barrier(0x7);  // no memory access sinks below: they run under the softmax
+        if (kj < 4 * KPL || (a.causal && j0 + kj > qw + 1)) {
+#pragma unroll
+            for (int e = 0; e < KPL; e++) {
+                const uint32_t kk = (uint32_t)(KPL * G + e);
+                if (kk >= kj || (a.causal && j0 + kk > i)) p[e] = MASKED;
+            }
+        }
+        // online softmax and psi_P (:264-342)
+        float rowmax = MASKED;
+#pragma unroll
+        for (int e = 0; e < KPL; e++) rowmax = fmaxf(rowmax, p[e]);
+        rowmax = ref_max4(rowmax);
+        const float m_new = rowmax > m ? rowmax : m;
+        const bool live = !(m_new < MASKED * 0.5f);
+        // not live: every argument is below -1e38 and its exp 0, as the
+        // reference sets alpha and p there (a NaN score's too, below)
+        const float mref = live ? m_new : 0.0f;
+        const float alpha = qbk_expf_neg(m - mref);
+#pragma unroll
+        for (int e = 0; e < KPL; e++) p[e] = qbk_expf_neg(p[e] - mref);
+        if (!__all(live)) {
+#pragma unroll
+            for (int e = 0; e < KPL; e++) p[e] = live ? p[e] : 0.0f;
+        }
+        const float esum = ref_ordered_sum<KPL>(p);
+        ref_i32x4_t pf[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            pf[j] = ref_i32x4_t{0, 0, 0, 0};
+#pragma unroll
+            for (int w = 0; w < (KPL < 16 ? KPL / 4 : 4); w++) {
+                // rint(127 p), 0 <= p <= 1, in the low byte of 127 p + 1.5 2^23 (a NaN
+                // p makes the row's ell, and so its outputs, NaN whatever its code)
+                uint32_t c4[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) c4[e] = __float_as_uint(p[16 * j + 4 * w + e] * 127.0f + 12582912.0f);
+                pf[j][w] = (int)__builtin_amdgcn_perm(__builtin_amdgcn_perm(c4[3], c4[2], 0x0c0c0400u),
+                                                      __builtin_amdgcn_perm(c4[1], c4[0], 0x0c0c0400u), 0x05040100u);
+            }
+        }
+        // O = alpha*O + (P^ V^) * (1/127) * dv  (:344-381); a query whose key
+        // blocks have ended (its wave's others go on) keeps its O, ell and m
+        const bool act = kb < kb_lane, all = kb < kb_first && __all(live);
+        ref_i32x4_t pv[NV];
+#pragma unroll
+        for (int ct = 0; ct < NV; ct++) {
+            pv[ct] = ref_i32x4_t{0, 0, 0, 0};
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+                pv[ct] = __builtin_amdgcn_mfma_i32_16x16x64_i8(vf[j][ct], pf[j], pv[ct], 0, 0, 0);
+        }
+        if (all) {
+#pragma unroll
+            for (int ct = 0; ct < NV; ct++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    o[ct][e] = alpha * o[ct][e] + (float)pv[ct][e] * (1.0f / 127.0f) * dl[ct][e];
+        } else {
+            // (selects by bits, not branches: v is 0 or all ones)
+            const uint32_t lv = live ? 0xffffffffu : 0u, av = act ? 0xffffffffu : 0u;
+#pragma unroll
+            for (int ct = 0; ct < NV; ct++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float prev = __uint_as_float(__float_as_uint(o[ct][e]) & lv);
+                    const float on = alpha * prev + (float)pv[ct][e] * (1.0f / 127.0f) * dl[ct][e];
+                    o[ct][e] = __uint_as_float((__float_as_uint(on) & av) | (__float_as_uint(o[ct][e]) & ~av));
+                }
+        }
+        if (act) {
+            ell = alpha * ell + esum;
+            m = m_new;
+        }
+    }
+    if (i >= S) return;
+    float *orow = a.out + ((size_t)bh * a.S + i) * a.dv;
+#pragma unroll
+    for (int ct = 0; ct < NV; ct++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const uint32_t c = (uint32_t)(16 * ct + 4 * G + e);
+            if (c < dv) orow[c] = o[ct][e] / ell;
+        }
+}
+
+// The keys a lane of sage_ref_tile holds for blocks of `block` keys, or 0
+// where sage_ref_main runs instead: blocks past 128 keys or head dims past
+// 128 would need more score or accumulator registers than a wave has.
+static int ref_tile_kpl(const RefArgs &a) {
+    if (a.d > 128 || a.dv > 128 || a.S > 0x7FFFFFFFu) return 0;
+    const size_t keys = a.block < a.S ? a.block : a.S;
+    return keys <= 16 ? 4 : keys <= 32 ? 8 : keys <= 64 ? 16 : keys <= 128 ? 32 : 0;
+}
+
+static int ref_tile_launch(const RefArgs &a, hipStream_t st) {
+    const size_t BH = a.B * a.H, grid = div_ceil(a.S, REF_TILE_Q) * BH;
+    if (grid > 0x7FFFFFFFu) return fail(QBK_ERR_VALIDATION, "sage attention: too many query tiles for one launch");
+    const uint32_t hpx = BH % 8 == 0 ? (uint32_t)(BH / 8) : 0;
+    const bool small = a.nv == 4;
+#define REF_TILE(K)                                                                                           \
+    if (small)                                                                                                \
+        hipLaunchKernelGGL((sage_ref_tile<K, 1, 4>), dim3((unsigned)grid), dim3(256), 0, st, a, hpx);         \
+    else                                                                                                      \
+        hipLaunchKernelGGL((sage_ref_tile<K, 2, 8>), dim3((unsigned)grid), dim3(256), 0, st, a, hpx);
+    switch (a.kpl) {
+        case 4: REF_TILE(4) break;
+        case 8: REF_TILE(8) break;
+        case 16: REF_TILE(16) break;
+        default: REF_TILE(32) break;
+    }
+#undef REF_TILE
+    QBK_HIP(hipGetLastError());
+    return QBK_OK;
+}
+
 static std::string shape_debug(const qbk_attn_shape *s) {
     return fmt("AttentionShape { batch: %zu, n_heads: %zu, n_kv_heads: %zu, seq_q: %zu, seq_kv: "
                "%zu, head_dim: %zu, val_dim: %zu }",
@@ -576,6 +1001,13 @@ static RefPlan ref_plan(const qbk_attn_shape *s, size_t block) {
     a.pst = a.S;
     a.pnkb = a.nkb;
     a.kb0 = 0;
+    const int kpl = ref_tile_kpl(a);
+    if (kpl) {  // whole MFMA steps (zero codes past d) of whole fragments
+        const bool small = a.d <= 64 && a.dv <= 64;
+        a.d4 = small ? 16 : 32;
+        a.kpl = (uint32_t)kpl;
+        a.nv = small ? 4 : 8;
+    }
     const size_t rows = a.B * a.H * a.S, bk = a.B * a.Hk;
     size_t off = 0;
     auto take = [&](size_t n) {
@@ -585,9 +1017,13 @@ static RefPlan ref_plan(const qbk_attn_shape *s, size_t block) {
     };
     P.off_kmean = take(bk * a.nkb * a.d * 4);
     P.off_kdelta = take(bk * a.S * 4);
-    P.off_khat = take(bk * a.S * a.d4 * 4);
+    P.off_khat = take(kpl ? bk * a.nkb * 4 * kpl * a.d4 * 4 : bk * a.S * a.d4 * 4);
     P.off_vd = take(bk * a.nkb * a.dv * 4);
-    P.off_vhat = take(bk * a.nkb * a.dv * a.blk4 * 4);
+    P.off_vhat = take(kpl ? bk * a.nkb * 16 * a.nv * 4 * kpl : bk * a.nkb * a.dv * a.blk4 * 4);
+    if (kpl) {  // nothing per row; a tile's last loads may run past the deltas by a block's worth of keys
+        P.ws_bytes = off + 512;
+        return P;
+    }
     P.off_gsc = take(a.sc_lds ? 0 : a.blk4 * 4 * rows * 4);
     P.off_gph = take(a.sc_lds ? 0 : a.blk4 * rows * 4);
     P.off_gpv = take(block > REF_CH ? a.dv * rows * 4 : 0);
@@ -615,13 +1051,14 @@ static int run_ref(const qbk_attn_shape *s, const float *q, const float *k, cons
     a.khat = (uint32_t *)(w + P.off_khat);
     a.vd = (float *)(w + P.off_vd);
     a.vhat = (uint32_t *)(w + P.off_vhat);
+    hipLaunchKernelGGL(sage_ref_prep, dim3((unsigned)a.nkb, (unsigned)(a.B * a.Hk), 2), dim3(256),
+                       ref_prep_lds(a.d, a.dv, a.block), st, a);
+    QBK_HIP(hipGetLastError());
+    if (a.kpl) return ref_tile_launch(a, st);
     a.gsc = (float *)(w + P.off_gsc);
     a.gph = (uint32_t *)(w + P.off_gph);
     a.gpv = (int *)(w + P.off_gpv);
     a.gout = (float *)(w + P.off_gout);
-    hipLaunchKernelGGL(sage_ref_prep, dim3((unsigned)a.nkb, (unsigned)(a.B * a.Hk)), dim3(256),
-                       ref_prep_lds(a.d, a.dv, a.block), st, a);
-    QBK_HIP(hipGetLastError());
     hipLaunchKernelGGL(sage_ref_main, dim3((unsigned)div_ceil(a.S, REF_ROWS), (unsigned)(a.B * a.H)),
                        dim3(REF_ROWS), P.lds_bytes, st, a);
     QBK_HIP(hipGetLastError());
