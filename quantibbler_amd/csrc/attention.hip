@@ -12,14 +12,18 @@
 // is 0/0 = NaN, as the NumPy reference's is.  Same validation, messages and
 // u32 index ceiling as the reference's face.
 //
-// One workgroup per (batch, head, query row): the row's query in LDS, keys
+// att_tile (below) serves head dims up to 128 on the f32 matrix cores; other
+// shapes run att_exact, one workgroup per (batch, head, query row): the
+// row's query in LDS, keys
 // in chunks of ATT_CHUNK -- a thread per key for the scores (dot products in
 // 16-channel partial sums), the chunk's max and sum by workgroup reductions,
 // an online softmax across chunks in f32, and a thread per output channel
 // summing p_j v[j][c] over the chunk's keys in 32-key partial sums (blocked
-// sums keep f32 rounding growing with the square root of the length).  Not a hot path: it is
+// sums keep f32 rounding growing with the square root of the length).  It is
 // what the quantised schemes are measured against.
 #include <math.h>
+
+#include <type_traits>
 
 #include "qbk_internal.h"
 
@@ -41,6 +45,7 @@ struct AttArgs {
     // between kv heads (head-major (B, Hkv, Skv, d): d and Skv d; a decoder
     // block's row-major cache (rows, Hkv d): Hkv d and d)
     size_t k_tok, k_head, v_tok, v_head;
+    uint32_t BH;  // att_tile: batches times heads
 };
 
 __device__ __forceinline__ float att_block_max(float v, float *red) {
@@ -134,6 +139,346 @@ __global__ void __launch_bounds__(ATT_THREADS) att_exact(AttArgs a) {
     }
 }
 
+// ---- the same on the f32 matrix cores --------------------------------------
+//
+// att_exact's arithmetic in f32 throughout, for head and value dims of at
+// most 128 whose rows take 16-byte loads.  A query row a workgroup reads every
+// key and value once per query, and a thread per key walks its key's row
+// alone; here a wave takes 16 QT queries of one head against 32 keys at a
+// time on v_mfma_f32_16x16x4_f32 (f32 products and sums), and the waves of a
+// workgroup split the keys (tiles of 32 round robin), so that a few queries
+// over many keys fill the chip as well; each keeps its own running max, sum
+// and output, merged through LDS at the end.
+//   S = K Q^T: A row = key, B column = query; a lane's float4 of channels
+//     16 s + 4 G .. feeds four MFMAs, of both operands.  Lane (col, G) gets
+//     keys 4 G .. 4 G + 3 of a 16-key tile for query col;
+//   O^T += V^T P^T: MFMA i of a tile takes keys 4 G + i, whose p are lane
+//     (col, G)'s i-th: P never leaves its lane.  A lane's float4 of channels
+//     64 h + 4 m .. feeds four MFMAs, whose outputs leave lane (col, G) the
+//     16 consecutive channels 64 h + 16 G .. of query col.
+// The sums stay blocked as in att_exact: a score in 16-channel partial sums,
+// the output in sums over 32 keys added to the running one.
+// A masked key's p is 0 and its value is not to be touched (0 x inf): tiles
+// that hold masked keys and a value that is not finite go key by key
+// (att_tile_masked), all others through the MFMAs.
+// What bounds it: the operands' way into registers (a 1 KB wave load takes
+// about 40 cycles of the CU's, which the f32 MFMAs, 32 cycles each for 2048
+// FLOP, only half cover: without the loads 2 x 777 queries run at 154 TFLOP/s,
+// the card's f32 rate).  Measured: 16 / 8 heads, 777 queries over 1300 keys,
+// d 128, causal: 5.34 ms with a row a workgroup, 0.11 ms here; one query of
+// 32 / 8 heads over 700 keys 130 -> 28 us.
+#define ATT_TILE_K 32  // keys a wave takes at a time
+#define ATT_WAVES 8    // waves a workgroup, the key tiles among them
+
+typedef float att_f32x4_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ float att_max4(float v) {  // over lanes l, l ^ 16, l ^ 32, l ^ 48
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    const float m = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float att_sum4(float v) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    const float m = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+// One tile's part of O for 16 queries, key by key: keys a query does not see
+// add nothing, whatever their values.  p of key 16 kt + 4 G + i is in lane
+// (col, G).
+template <int NH>
+__device__ __forceinline__ void att_tile_masked(const float *vb, size_t v_tok, uint32_t dv, uint32_t j0, uint32_t kend_wg,
+                                             uint32_t kend, const float p[ATT_TILE_K / 4], int lane,
+                                             att_f32x4_t (*part)[4]) {
+    const int col = lane & 15, G = lane >> 4;
+    for (int hh = 0; hh < NH; hh++)
+        for (int j = 0; j < 4; j++) part[hh][j] = att_f32x4_t{0, 0, 0, 0};
+    for (uint32_t kk = 0; kk < ATT_TILE_K && j0 + kk < kend_wg; kk++) {
+        float pk = 0.0f;
+#pragma unroll
+        for (int e = 0; e < ATT_TILE_K / 4; e++)
+            if ((uint32_t)e == 4 * (kk / 16) + kk % 4) pk = p[e];
+        pk = __shfl(pk, col + 16 * (int)(kk % 16 / 4), 64);
+        const bool see = j0 + kk < kend;
+        const float *vr = vb + (size_t)(j0 + kk) * v_tok;
+        for (int hh = 0; hh < NH; hh++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t c = 64 * hh + 16 * G + 4 * i;
+                if (c >= dv) continue;
+                const att_f32x4_t v = *(const att_f32x4_t *)(vr + c);
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (see) part[hh][j][i] += pk * v[j];
+            }
+    }
+}
+
+// DT: 16-channel steps of the head dim; NH: 64-channel halves of the value
+// dim; QW: 16-query tiles of a workgroup, its other waves splitting the keys.
+template <int DT, int NH, int QW>
+__global__ void __launch_bounds__(64 * ATT_WAVES, 2) att_tile(AttArgs a) {
+    constexpr int KT = ATT_TILE_K / 16, KW = ATT_WAVES / QW;
+    __shared__ float ml[2][ATT_WAVES][16];
+    __shared__ __attribute__((aligned(16))) float ob[ATT_WAVES][16][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, G = lane >> 4, qw = wave % QW, kw = wave / QW;
+    // the longest key ranges first, heads innermost
+    const uint32_t BH = a.BH, nq = (uint32_t)((a.Sq + 16 * QW - 1) / (16 * QW));
+    const uint32_t bh = blockIdx.x % BH, qi = nq - 1 - blockIdx.x / BH;
+    const size_t b = bh / a.H, h = bh % a.H;
+    const size_t bk = b * a.Hk + h / (a.H / a.Hk);
+    const uint32_t Sq = (uint32_t)a.Sq, Skv = (uint32_t)a.Skv, d = (uint32_t)a.d, dv = (uint32_t)a.dv;
+    const uint32_t qg = qi * (16 * QW), q0 = qg + 16 * qw;  // the workgroup's first query, the wave's
+    const float *kb = a.k + bk * a.k_head, *vb = a.v + bk * a.v_head;
+    // keys visible to query i: j < i + 1 + Skv - Sq (none below 0)
+    auto visible = [&](uint32_t i) {
+        if (!a.causal) return Skv;
+        const int64_t e = (int64_t)i + 1 + Skv - Sq;
+        return e < 0 ? 0u : e < (int64_t)Skv ? (uint32_t)e : Skv;
+    };
+    const uint32_t qlast = q0 + 15 < Sq ? q0 + 15 : Sq - 1;
+    const uint32_t kend_wg = q0 < Sq ? visible(qlast) : 0, kend_min = visible(q0);
+    const uint32_t iq = q0 + col < Sq ? q0 + col : Sq - 1;  // past the last: it repeats the last one, stores nothing
+    const uint32_t kend = visible(iq);
+    att_f32x4_t qf[DT];
+    {
+        const float *qr = a.q + ((size_t)bh * a.Sq + iq) * a.d;
+#pragma unroll
+        for (int s = 0; s < DT; s++) {
+            qf[s] = *(const att_f32x4_t *)(qr + (16u * s < d ? 16 * s : 0) + 4 * G);
+        }
+    }
+    att_f32x4_t o[NH][4];
+    float m = -INFINITY, l = 0.0f;
+#pragma unroll
+    for (int hh = 0; hh < NH; hh++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) o[hh][j] = att_f32x4_t{0, 0, 0, 0};
+    // Rows are addressed from a uniform pointer (scalar registers) plus one
+    // lane offset; a tile that runs past the range (its last) clamps each
+    // lane's row to the range's last.  Keys load a tile ahead, under the
+    // P V MFMAs.
+    const uint32_t k_tok = (uint32_t)a.k_tok, v_tok = (uint32_t)a.v_tok;
+    uint32_t vc[NH];  // this lane's first channel of a half (channels past dv repeat the first)
+#pragma unroll
+    for (int hh = 0; hh < NH; hh++) vc[hh] = 64u * hh + 4 * col < dv ? 64 * hh + 4 * col : 0;
+    att_f32x4_t kf[KT][DT];
+    auto load_k = [&](uint32_t j0) {
+        const uint32_t last = kend_wg - 1 - j0;  // >= 0: the tile's first key is in the range
+#pragma unroll
+        for (int kt = 0; kt < KT; kt++) {
+            const uint32_t row = 16 * kt + col;
+            const float *kt0 = kb + (size_t)j0 * k_tok;
+            const uint32_t off = (row < last ? row : last) * k_tok + 4 * G;
+#pragma unroll
+            for (int s = 0; s < DT; s++)
+                kf[kt][s] = *(const att_f32x4_t *)(kt0 + (16u * s < d ? 16 * s : 0) + off);
+        }
+    };
+    // One tile.  edge: some of its keys are masked for some query.  The keys
+    // of the tile at jn load under the P V MFMAs (jn past the range: none).
+    auto tile = [&](uint32_t j0, uint32_t jn, auto edge) {
+        // values of the tile's keys, under the S MFMAs
+        att_f32x4_t vf[KT][4][NH];
+        {
+            const uint32_t last = kend_wg - 1 - j0;
+            const float *vt0 = vb + (size_t)j0 * v_tok;
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const uint32_t row = 16 * kt + 4 * G + i;
+                    const uint32_t off = (row < last ? row : last) * v_tok;
+#pragma unroll
+                    for (int hh = 0; hh < NH; hh++) vf[kt][i][hh] = *(const att_f32x4_t *)(vt0 + off + vc[hh]);
+                }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float p[4 * KT];
+        {
+            att_f32x4_t acc[KT];
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++) acc[kt] = att_f32x4_t{0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < DT; s++)
+                if (16u * s < d) {
+                    att_f32x4_t sp[KT];  // 16-term partial sums, as att_exact's
+#pragma unroll
+                    for (int kt = 0; kt < KT; kt++) sp[kt] = att_f32x4_t{0, 0, 0, 0};
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+#pragma unroll
+                        for (int kt = 0; kt < KT; kt++)
+                            sp[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kt][s][e], qf[s][e], sp[kt], 0, 0, 0);
+#pragma unroll
+                    for (int kt = 0; kt < KT; kt++) acc[kt] += sp[kt];
+                }
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) p[4 * kt + e] = acc[kt][e] * a.scale;
+        }
+        if (!edge) load_k(jn);
+        __builtin_amdgcn_sched_barrier(0);
+        bool slow = false;
+        if constexpr (edge) {
+#pragma unroll
+            for (int e = 0; e < 4 * KT; e++)
+                if (j0 + 16 * (e / 4) + 4 * G + e % 4 >= kend) p[e] = -INFINITY;
+            bool fin = true;
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int hh = 0; hh < NH; hh++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) fin = fin & (fabsf(vf[kt][i][hh][e]) < INFINITY);
+            slow = !__all(fin);
+        }
+        float cmax = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 4 * KT; e++) cmax = fmaxf(cmax, p[e]);
+        const float mn = fmaxf(m, att_max4(cmax));
+        if (__any(mn != m)) {  // some query's max moved
+            const float alpha = m == -INFINITY ? 0.0f : expf(m - mn);
+            l *= alpha;
+#pragma unroll
+            for (int hh = 0; hh < NH; hh++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) o[hh][j] *= alpha;
+            m = mn;
+        }
+        float part = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4 * KT; e++) {
+            const float x = expf(p[e] - mn);
+            p[e] = p[e] == -INFINITY ? 0.0f : x;
+            part += p[e];
+        }
+        l += part;
+        if constexpr (edge) {
+            if (slow) {
+                att_f32x4_t sum[NH][4];
+                att_tile_masked<NH>(vb, a.v_tok, dv, j0, kend_wg, kend, p, lane, sum);
+#pragma unroll
+                for (int hh = 0; hh < NH; hh++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) o[hh][j] += sum[hh][j];
+                return;
+            }
+        }
+#pragma unroll
+        for (int hh = 0; hh < NH; hh++) {
+            att_f32x4_t sum[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) sum[j] = att_f32x4_t{0, 0, 0, 0};
+#pragma unroll
+            for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        sum[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[kt][i][hh][j], p[4 * kt + i], sum[j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < 4; j++) o[hh][j] += sum[j];
+        }
+    };
+    // the tiles every query sees in full, then the edge's (two at most)
+    uint32_t j0 = kw * ATT_TILE_K;
+    if (j0 + ATT_TILE_K <= kend_min) {
+        load_k(j0);
+        for (; j0 + ATT_TILE_K <= kend_min; j0 += KW * ATT_TILE_K) {
+            const uint32_t jn = j0 + KW * ATT_TILE_K;
+            tile(j0, jn < kend_wg ? jn : j0, std::false_type{});
+        }
+    }
+    for (; j0 < kend_wg; j0 += KW * ATT_TILE_K) {
+        load_k(j0);
+        tile(j0, 0, std::true_type{});
+    }
+    // merge the waves: every wave's output and sum on the largest max
+    const float ls = att_sum4(l);
+    if (G == 0) {
+        ml[0][wave][col] = m;
+        ml[1][wave][col] = ls;
+    }
+    __syncthreads();
+    float f;
+    {
+        float M = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < KW; w++) M = fmaxf(M, ml[0][w * QW + qw][col]);
+        f = m == -INFINITY ? 0.0f : expf(m - M);
+    }
+#pragma unroll
+    for (int hh = 0; hh < NH; hh++) {
+        if (hh) __syncthreads();  // the first half's sums are read
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            att_f32x4_t v;
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = o[hh][j][i] * f;
+            *(att_f32x4_t *)&ob[wave][col][16 * G + 4 * i] = v;
+        }
+        __syncthreads();
+        for (int x = tid; x < QW * 16 * 64; x += 64 * ATT_WAVES) {
+            const int t = x / 1024, q = x / 64 % 16, c = x % 64;
+            const uint32_t i = qg + 16 * t + q;
+            if (i >= Sq || 64u * hh + c >= dv) continue;
+            float M = -INFINITY, L = 0.0f, sum = 0.0f;
+#pragma unroll
+            for (int w = 0; w < KW; w++) M = fmaxf(M, ml[0][w * QW + t][q]);
+#pragma unroll
+            for (int w = 0; w < KW; w++) {
+                const float mw = ml[0][w * QW + t][q];
+                L += ml[1][w * QW + t][q] * (mw == -INFINITY ? 0.0f : expf(mw - M));
+                sum += ob[w * QW + t][q][c];
+            }
+            a.out[((size_t)bh * a.Sq + i) * a.dv + 64 * hh + c] = sum / L;
+        }
+    }
+}
+
+// Whether att_tile serves the call: 16-byte rows of queries, keys and values.
+static bool att_tile_fits(const AttArgs &a) {
+    return a.d <= 128 && a.dv <= 128 && (a.d | a.dv) % 16 == 0 && (a.k_tok | a.v_tok | a.k_head | a.v_head) % 4 == 0 &&
+           a.k_tok <= 0x1000000u && a.v_tok <= 0x1000000u &&
+           (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) & 15) == 0 && a.Sq <= 0x40000000u &&
+           a.Skv <= 0x40000000u;
+}
+
+static int att_tile_launch(AttArgs a, size_t B, hipStream_t st) {
+    a.BH = (uint32_t)(B * a.H);
+    // More query tiles a workgroup share each key's and value's way through
+    // the L1 but leave fewer workgroups: 16 / 8 heads, d 128, 1300 keys (us
+    // for 1, 2, 4 tiles): 777 queries causal 124, 107, 127; 2 x 777 not causal
+    // 291, 279, 255; 400 queries of d 80 over 700 keys 56, 47, 47; 64 queries
+    // 44 each.
+    const int qw = div_ceil(a.Sq, 64) * B * a.H >= 400 ? 4 : div_ceil(a.Sq, 32) * B * a.H >= 150 ? 2 : 1;
+    const size_t grid = div_ceil(a.Sq, 16 * (size_t)qw) * B * a.H;
+    if (grid > 0x7FFFFFFFull) return fail(QBK_ERR_VALIDATION, "attention: too many query tiles for one launch");
+    const bool small = a.d <= 64 && a.dv <= 64;
+#define ATT_GO(QW)                                                                                        \
+    if (small)                                                                                            \
+        hipLaunchKernelGGL((att_tile<4, 1, QW>), dim3((unsigned)grid), dim3(64 * ATT_WAVES), 0, st, a);   \
+    else                                                                                                  \
+        hipLaunchKernelGGL((att_tile<8, 2, QW>), dim3((unsigned)grid), dim3(64 * ATT_WAVES), 0, st, a);
+    if (qw == 4) {
+        ATT_GO(4)
+    } else if (qw == 2) {
+        ATT_GO(2)
+    } else {
+        ATT_GO(1)
+    }
+#undef ATT_GO
+    QBK_HIP(hipGetLastError());
+    return QBK_OK;
+}
+
 // gpu_attention.rs:466-509: validation in the reference's order and words,
 // then the u32 index ceiling of its device face.
 static int validate_exact(const qbk_attn_shape *s, const size_t *lens) {
@@ -178,6 +523,7 @@ static int launch_exact(const qbk_attn_shape *s, const float *q, const float *k,
               s->seq_kv * s->val_dim};
     const size_t rows = s->batch * s->n_heads * s->seq_q;
     if (rows > 0x7FFFFFFFull) return fail(QBK_ERR_VALIDATION, "attention: too many query rows for one launch");
+    if (att_tile_fits(a)) return att_tile_launch(a, s->batch, st);
     hipLaunchKernelGGL(att_exact, dim3((unsigned)rows), dim3(ATT_THREADS), 0, st, a);
     QBK_HIP(hipGetLastError());
     return QBK_OK;
@@ -192,6 +538,7 @@ int attention_exact_cache(const float *q, const float *kc, const float *vc, size
     if (rows == 0 || H == 0 || Hk == 0 || H % Hk != 0 || hd == 0 || hd > ATT_MAXD)
         return fail(QBK_ERR_VALIDATION, "exact cache attention: bad shape");
     AttArgs a{q, kc, vc, out, H, Hk, 1, rows, hd, hd, 0, 1.0f / sqrtf((float)hd), Hk * hd, hd, Hk * hd, hd};
+    if (att_tile_fits(a)) return att_tile_launch(a, 1, st);
     hipLaunchKernelGGL(att_exact, dim3((unsigned)H), dim3(ATT_THREADS), 0, st, a);
     QBK_HIP(hipGetLastError());
     return QBK_OK;
