@@ -40,6 +40,7 @@ CFLAGS = [
 EXTRA = {
     "decode.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "serve64.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 
 

@@ -54,8 +54,7 @@ struct qbk_block {
     std::vector<size_t> filled;  // per sequence: cache rows holding its keys and values
     int face;                    // QBK_ATTN_SAGE (the sage decode attention) or QBK_ATTN_EXACT
     int serving;                 // QBK_BF16, or QBK_F32 (apply's f64 products, f32 norms)
-    float *xf;                   // fp32 serving: the normalised row, f32 [d] (null until set)
-    double *f64s;                // fp32 serving: the f64 products' scratch
+    double *f64s;                // fp32 serving: the f64 products' scratch (null until set)
     // per-call buffers
     uint16_t *xcat;           // bf16 [3 d] (q, k, v inputs), then [2 d] (gate, up)
     float *ycat;              // f32 [(H + 2 Hk) hd], then [2 ffn]
@@ -105,10 +104,24 @@ __global__ void __launch_bounds__(BLKD_NORM_THREADS) blkd_norm(const float *a, c
     }
 }
 
+// The layers that a vector feeds at fp32 serving: each one's s2 and where its
+// z = f64(s2 x) goes (serve64.hip, f64_pos order; n is a multiple of 128 or
+// the rest of the last 128 is zero).
+struct BlkdZ {
+    const float *s2[F64_MAXL];
+    double *z[F64_MAXL];
+};
+__device__ __forceinline__ void blkd_put_z(const BlkdZ &o, int nl, int i, float x, bool valid) {
+#pragma unroll
+    for (int l = 0; l < F64_MAXL; l++)
+        if (l < nl) o.z[l][f64_pos((uint32_t)i)] = valid ? (double)(o.s2[l][i] * x) : 0.0;
+}
+
 // blkd_norm at fp32 serving (norm_apply's Fp32 arm, engine/mod.rs:837-852):
-// x = RMS-normalised hsum times w in f32, no bf16 roundings; x f32 [d].
-__global__ void __launch_bounds__(BLKD_NORM_THREADS) blkd_norm_f32(const float *a, const float *r, float *hout,
-                                                                  const float *w, float eps, float *x, int d) {
+// x = RMS-normalised hsum times w in f32, no bf16 roundings, written as the
+// z of the nl projections it feeds.
+__global__ void __launch_bounds__(BLKD_NORM_THREADS) blkd_norm_z(const float *a, const float *r, float *hout,
+                                                                const float *w, float eps, BlkdZ o, int nl, int d) {
     __shared__ float red[BLKD_NORM_THREADS / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     float ss = 0.0f;
@@ -119,17 +132,34 @@ __global__ void __launch_bounds__(BLKD_NORM_THREADS) blkd_norm_f32(const float *
         ss += v * v;
     }
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
+    for (int o2 = 32; o2 >= 1; o2 >>= 1) ss += __shfl_xor(ss, o2, 64);
     if (lane == 0) red[wave] = ss;
     __syncthreads();
     float tot = 0.0f;
     for (int i = 0; i < BLKD_NORM_THREADS / 64; i++) tot += red[i];
     const float inv = 1.0f / sqrtf(tot / (float)d + eps);
-    for (int i = tid; i < d; i += BLKD_NORM_THREADS) {
-        float v = a[i];
-        if (r) v = v + r[i];
-        x[i] = v * inv * w[i];
+    for (int i = tid; i < ((d + 127) & ~127); i += BLKD_NORM_THREADS) {
+        float v = 0.0f;
+        if (i < d) {
+            v = a[i];
+            if (r) v = v + r[i];
+            v = v * inv * w[i];
+        }
+        blkd_put_z(o, nl, i, v, i < d);
     }
+}
+
+// hidden = g u / (1 + exp(-g)) as blkd_swiglu, written as the down
+// projection's z
+__global__ void blkd_swiglu_z(const float *gu, BlkdZ o, int ffn) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= ((ffn + 127) & ~127)) return;
+    float hid = 0.0f;
+    if (i < ffn) {
+        const float g = gu[i], u = gu[ffn + i];
+        hid = g * u / (1.0f + expf(0.0f - g));
+    }
+    blkd_put_z(o, 1, i, hid, i < ffn);
 }
 
 // Per-head RMSNorm (optional) and RoPE of q and k at position pos: one wave
@@ -689,7 +719,6 @@ int qbk_block_create_seqs(qbk_ctx *ctx, const qbk_factor *const *layers, const f
     B->nseq = n_seqs;
     B->face = QBK_ATTN_SAGE;
     B->serving = QBK_BF16;
-    B->xf = nullptr;
     B->f64s = nullptr;
     B->tokens.assign(n_seqs, 0);
     B->filled.assign(n_seqs, 0);
@@ -786,18 +815,25 @@ static const char *const kF32Only =
 // ServingDtype::Fp32): norms in f32 without bf16 roundings (:837-876), the
 // seven projections as apply's f64 products (:393-436), q/k norms and RoPE,
 // the cache append, the block's attention face over rows 0 .. pos, SwiGLU,
-// the residuals.  A parity face: a few launches a projection.
+// the residuals.  Projections of one input run in one pair of launches; the
+// norms and SwiGLU write the z of the projections they feed, the down
+// projection adds the residual.
 static int block_decode_f32(qbk_ctx *ctx, qbk_block *B, float *h, size_t pos, hipStream_t s) {
     int rc;
     const int d = (int)B->d, hd = (int)B->hd, H = (int)B->H, Hk = (int)B->Hk, ffn = (int)B->ffn;
-    auto proj = [&](int li, const float *x, float *y) {
-        return factor_apply_f64_dev(ctx, B->lay[li], x, y, B->f64s, s);
+    auto feeds = [&](const qbk_factor *const *L, int n) {
+        BlkdZ o{};
+        for (int i = 0; i < n; i++) {
+            o.s2[i] = L[i]->s2;
+            o.z[i] = factor_f64_z(L, i, B->f64s);
+        }
+        return o;
     };
-    hipLaunchKernelGGL(blkd_norm_f32, dim3(1), dim3(BLKD_NORM_THREADS), 0, s, h, (const float *)nullptr,
-                       (float *)nullptr, B->w_in, B->eps, B->xf, d);
+    hipLaunchKernelGGL(blkd_norm_z, dim3(1), dim3(BLKD_NORM_THREADS), 0, s, (const float *)h, (const float *)nullptr,
+                       (float *)nullptr, (const float *)B->w_in, B->eps, feeds(B->lay, 3), 3, d);
     QBK_HIP(hipGetLastError());
-    float *q = B->ycat, *k = q + (size_t)H * hd, *v = k + (size_t)Hk * hd;
-    if ((rc = proj(0, B->xf, q)) || (rc = proj(1, B->xf, k)) || (rc = proj(2, B->xf, v))) return rc;
+    float *const qkv[3] = {B->ycat, B->ycat + (size_t)H * hd, B->ycat + (size_t)(H + Hk) * hd};
+    if ((rc = factor_f64_staged(B->lay, 3, qkv, nullptr, B->f64s, s))) return rc;
     hipLaunchKernelGGL(blkd_qk_rope<true>, dim3(H + Hk), dim3(64), 0, s, B->ycat, B->rope, pos,
                        (const uint32_t *)nullptr, B->cap, B->w_q, B->w_k, B->eps, B->qrot, B->kc, B->vc, H, Hk, hd);
     QBK_HIP(hipGetLastError());
@@ -813,17 +849,16 @@ static int block_decode_f32(qbk_ctx *ctx, qbk_block *B, float *h, size_t pos, hi
         B->tokens[0] = pos + 1;
     }
     B->filled[0] = pos + 1;
-    if ((rc = proj(3, B->attn, B->oout))) return rc;
-    hipLaunchKernelGGL(blkd_norm_f32, dim3(1), dim3(BLKD_NORM_THREADS), 0, s, B->oout, (const float *)h, B->h1,
-                       B->w_post, B->eps, B->xf, d);
+    float *const oo = B->oout, *const gu[2] = {B->ycat, B->ycat + ffn}, *const out = h;
+    if ((rc = factor_f64_run(B->lay + 3, 1, B->attn, &oo, B->f64s, s))) return rc;
+    hipLaunchKernelGGL(blkd_norm_z, dim3(1), dim3(BLKD_NORM_THREADS), 0, s, (const float *)B->oout, (const float *)h,
+                       B->h1, (const float *)B->w_post, B->eps, feeds(B->lay + 4, 2), 2, d);
     QBK_HIP(hipGetLastError());
-    if ((rc = proj(4, B->xf, B->ycat)) || (rc = proj(5, B->xf, B->ycat + ffn))) return rc;
-    hipLaunchKernelGGL(blkd_swiglu, dim3((ffn + 255) / 256), dim3(256), 0, s, B->ycat, B->hid, ffn);
+    if ((rc = factor_f64_staged(B->lay + 4, 2, gu, nullptr, B->f64s, s))) return rc;
+    hipLaunchKernelGGL(blkd_swiglu_z, dim3((unsigned)((ffn + 127) / 128)), dim3(128), 0, s, (const float *)B->ycat,
+                       feeds(B->lay + 6, 1), ffn);
     QBK_HIP(hipGetLastError());
-    if ((rc = proj(6, B->hid, B->dout))) return rc;
-    hipLaunchKernelGGL(blkd_add, dim3((d + 255) / 256), dim3(256), 0, s, B->dout, B->h1, h, d);
-    QBK_HIP(hipGetLastError());
-    return QBK_OK;
+    return factor_f64_staged(B->lay + 6, 1, &out, B->h1, B->f64s, s);  // h = down(hid) + h1
 }
 
 // The decode of one position of sequence 0: at pos (host), or with pos_dev
@@ -1024,20 +1059,17 @@ int qbk_block_set_serving(qbk_ctx *ctx, qbk_block *B, int serving) {
     if (!B) return fail(QBK_ERR_VALIDATION, "null block");
     if (serving != QBK_F32 && serving != QBK_BF16)
         return fail(QBK_ERR_VALIDATION, "serving dtype must be QBK_F32 or QBK_BF16");
-    if (serving == QBK_F32 && !B->xf) {
+    if (serving == QBK_F32 && !B->f64s) {
         if ((rc = bind(ctx))) return rc;
         if (B->device != ctx->device)
             return fail(QBK_ERR_VALIDATION, "block lives on another device than the context");
-        size_t nd = 0;
-        for (const qbk_factor *L : B->lay) nd = std::max(nd, L->din + L->r + L->dout);
-        void *xf = nullptr, *sc = nullptr;
-        QBK_HIP(hipMalloc(&xf, B->d * sizeof(float)));
-        B->allocs.push_back(xf);
+        const size_t nd = std::max(std::max(factor_f64_scratch(B->lay, 3), factor_f64_scratch(B->lay + 3, 1)),
+                                   std::max(factor_f64_scratch(B->lay + 4, 2), factor_f64_scratch(B->lay + 6, 1)));
+        void *sc = nullptr;
         QBK_HIP(hipMalloc(&sc, nd * sizeof(double)));
         B->allocs.push_back(sc);
         for (const qbk_factor *L : B->lay)
-            if ((rc = factor_rows_ready(L, nullptr))) return rc;
-        B->xf = (float *)xf;
+            if ((rc = factor_f64_ready(L, nullptr))) return rc;
         B->f64s = (double *)sc;
     }
     B->serving = serving;

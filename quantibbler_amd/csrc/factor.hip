@@ -11,8 +11,8 @@
 // in prefill.hip.
 //
 // A layer is uploaded once and repacked into three device layouts:
-//   * ref rows   : the engine's per-row bitplanes (ub_rows, vb_t_rows) for
-//                  the f64 serving path (sequential, bit-identical);
+//   * f64 words  : (16-row group, 128-k slice) blocks of 64 words for the
+//                  fp32 serving path (serve64.hip), formed on its first call;
 //   * q4 words   : (64-row group, 128-k slice) blocks of 64 lane x 4 words
 //                  in the fp4 operand order of the scaled MFMA (decode);
 //   * g32 words  : (128-row group, 64-k slice) blocks of 64 lane x 4 words,
@@ -90,27 +90,6 @@ static void container_to_rows_transposed(const uint8_t *packed, size_t din, size
             size_t b = j * r + k;
             if ((packed[b >> 3] >> (b & 7)) & 1) out[k * rw + (j >> 3)] |= (uint8_t)(1u << (j & 7));
         }
-}
-
-// The reference's per-row bitplanes (bit k of row i at byte k/8, LSB first,
-// set for +1) rebuilt from the fp4 decode layout: one thread per row byte,
-// each of its bits read from the word and bit repack_q4 put it at (the
-// inverse of kq4: k % 128 = 64 (g & 1) + 32 (e >> 4) + 16 (g >> 1) + e % 16).
-__global__ void q4_to_rows(const uint32_t *q4, size_t n_rows, size_t n_bits, size_t bits_q, uint8_t *rows) {
-    const size_t rw = (n_bits + 7) / 8, idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n_rows * rw) return;
-    const size_t i = idx / rw, j = idx % rw, ns = bits_q / 128;
-    const size_t rg = i / 64, rt = (i % 64) / 16, l15 = i % 16;
-    uint32_t byte = 0;
-    for (int b = 0; b < 8; b++) {
-        const size_t k = 8 * j + b;
-        if (k >= n_bits) break;
-        const uint32_t kk = (uint32_t)(k % 128), s = (uint32_t)(k / 128);
-        const uint32_t g = 2 * ((kk >> 4) & 1) + ((kk >> 6) & 1), e = 16 * ((kk >> 5) & 1) + (kk & 15);
-        const uint32_t w = q4[((rg * ns + s) * 64 + 16 * g + l15) * 4 + rt];
-        if (!((w >> (4 * (e & 7) + (e >> 3))) & 1)) byte |= 1u << b;
-    }
-    rows[idx] = (uint8_t)byte;
 }
 
 // v's fp16 bits when v is an fp16 value (zero, a normal or subnormal fp16
@@ -210,7 +189,7 @@ static int build_layer(qbk_ctx *ctx, size_t dout, size_t din, size_t r, const ui
         return rc;                                                         \
     }                                                                      \
     L->field = (decltype(L->field))p;
-    L->ub_rows = L->vbt_rows = nullptr;  // formed on the first f64-face call (q4_to_rows)
+    L->vt_f64 = L->u_f64 = nullptr;  // formed on the first fp32-serving call (serve64.hip)
     UP(vt_g32, vf.data(), vf.size() * 4);
     UP(u_g32, uf.data(), uf.size() * 4);
     UP(vt_q4, vq.data(), vq.size() * 4);
@@ -428,72 +407,6 @@ int qbk_factor_linear_noalloc_dev(qbk_ctx *ctx, const qbk_factor *L, const uint1
     return qbk_factor_linear_dev(ctx, L, x, batch, y, y_dtype, ws, need, stream);
 }
 
-// The f64 serving path's two elementwise ends (engine/mod.rs:419-436):
-// z = f64(s2 * x), an f32 product widened; y = f32(u) * s1 + b, a multiply
-// then an add (the file is built without contraction).
-__global__ void factor_f64_in(const float *x, const float *s2, double *z, size_t n) {
-    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (i < n) z[i] = (double)(s2[i] * x[i]);
-}
-
-__global__ void factor_f64_out(const double *u, const float *s1, const float *bias, float *y, size_t n) {
-    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (i < n) y[i] = ((float)u[i]) * s1[i] + bias[i];
-}
-
-}  // extern "C"
-
-namespace qbk {
-
-// The reference's row bitplanes of L (ub_rows, vbt_rows), formed from the
-// decode layout on first use and kept with the layer.
-int factor_rows_ready(const qbk_factor *L, hipStream_t s) {
-    static std::mutex mu;
-    std::lock_guard<std::mutex> lock(mu);
-    if (L->ub_rows) return QBK_OK;
-    qbk_factor *M = const_cast<qbk_factor *>(L);
-    void *pu = nullptr, *pv = nullptr;
-    const size_t nu = L->dout * div_ceil(L->r, 8), nv = L->r * div_ceil(L->din, 8);
-    QBK_HIP(hipMalloc(&pu, nu));
-    M->allocs.push_back(pu);
-    QBK_HIP(hipMalloc(&pv, nv));
-    M->allocs.push_back(pv);
-    hipLaunchKernelGGL(q4_to_rows, dim3((unsigned)div_ceil(nu, 256)), dim3(256), 0, s, L->u_q4, L->dout, L->r,
-                       L->r_q, (uint8_t *)pu);
-    QBK_HIP(hipGetLastError());
-    hipLaunchKernelGGL(q4_to_rows, dim3((unsigned)div_ceil(nv, 256)), dim3(256), 0, s, L->vt_q4, L->r, L->din,
-                       L->din_q, (uint8_t *)pv);
-    QBK_HIP(hipGetLastError());
-    QBK_HIP(hipStreamSynchronize(s));
-    M->vbt_rows = (uint8_t *)pv;
-    M->ub_rows = (uint8_t *)pu;
-    return QBK_OK;
-}
-
-// apply's fp32 serving (engine/mod.rs:393-436) of one token on the device:
-// z = f64(s2 x), t = Vb^T z and u = Ub t as f64 matvecs in element order
-// (the packed f64 product), y = f32(u) s1 + b.  x, y f32 device vectors;
-// scratch holds din + r + dout doubles; the rows must be formed
-// (factor_rows_ready).
-int factor_apply_f64_dev(qbk_ctx *ctx, const qbk_factor *L, const float *x, float *y, double *scratch,
-                         hipStream_t s) {
-    int rc;
-    double *z = scratch, *t = z + L->din, *u = t + L->r;
-    hipLaunchKernelGGL(factor_f64_in, dim3((unsigned)((L->din + 255) / 256)), dim3(256), 0, s, x,
-                       (const float *)L->s2, z, L->din);
-    QBK_HIP(hipGetLastError());
-    if ((rc = qbk_packed_matvec_dev(ctx, QBK_F64, L->vbt_rows, L->r, L->din, z, t, s))) return rc;
-    if ((rc = qbk_packed_matvec_dev(ctx, QBK_F64, L->ub_rows, L->dout, L->r, t, u, s))) return rc;
-    hipLaunchKernelGGL(factor_f64_out, dim3((unsigned)((L->dout + 255) / 256)), dim3(256), 0, s, (const double *)u,
-                       (const float *)L->s1, (const float *)L->bias, y, L->dout);
-    QBK_HIP(hipGetLastError());
-    return QBK_OK;
-}
-
-}  // namespace qbk
-
-extern "C" {
-
 // engine/mod.rs:393-460 apply / apply_bf16 with host buffers.
 int qbk_factor_apply(qbk_ctx *ctx, const qbk_factor *L, int serving, const float *x, size_t batch,
                      float *y) {
@@ -506,21 +419,20 @@ int qbk_factor_apply(qbk_ctx *ctx, const qbk_factor *L, int serving, const float
     CallStream cs;
     if ((rc = cs.create())) return rc;
     if (serving == QBK_F32) {
-        // per token: z = f64(s2*x), the two f64 matvecs in element order,
-        // y = f32(u)*s1 + b -- all on the device.  The matvecs read the
-        // reference's row layout, which the layer forms from its decode
+        // per token: z = f64(s2*x), the two f64 products in element order,
+        // y = f32(u)*s1 + b (serve64.hip); the layer forms that path's sign
         // layout on the first such call (a third copy of the signs only for
         // layers that use this face).
-        if ((rc = factor_rows_ready(L, cs.s))) return rc;
+        if ((rc = factor_f64_ready(L, cs.s))) return rc;
         DevBuf dx, dy, dsc;
         if ((rc = dx.alloc(batch * L->din * 4)) || (rc = dy.alloc(batch * L->dout * 4)) ||
-            (rc = dsc.alloc((L->din + L->r + L->dout) * 8)))
+            (rc = dsc.alloc(factor_f64_scratch(&L, 1) * 8)))
             return rc;
         QBK_HIP(hipMemcpyAsync(dx.p, x, batch * L->din * 4, hipMemcpyHostToDevice, cs.s));
-        for (size_t bb = 0; bb < batch; bb++)
-            if ((rc = factor_apply_f64_dev(ctx, L, (const float *)dx.p + bb * L->din, (float *)dy.p + bb * L->dout,
-                                           (double *)dsc.p, cs.s)))
-                return rc;
+        for (size_t bb = 0; bb < batch; bb++) {
+            float *yb = (float *)dy.p + bb * L->dout;
+            if ((rc = factor_f64_run(&L, 1, (const float *)dx.p + bb * L->din, &yb, (double *)dsc.p, cs.s))) return rc;
+        }
         QBK_HIP(hipMemcpyAsync(y, dy.p, batch * L->dout * 4, hipMemcpyDeviceToHost, cs.s));
         QBK_HIP(hipStreamSynchronize(cs.s));
         return QBK_OK;

@@ -48,8 +48,8 @@ struct qbk_factor {
     int device, num_cus;
     size_t dout, din, r;
     size_t din_p, r_p, dout_p;  // padded for the MFMA tiles (64 / 128 / 128)
-    uint8_t *ub_rows, *vbt_rows;      // reference per-row bitplanes, formed from the decode layout on the
-                                      // first f64-face call (null until then)
+    uint32_t *vt_f64, *u_f64;         // serve64.hip's sign layout, formed from the decode layout on the first
+                                      // fp32-serving call (null until then)
     uint32_t *vt_g32, *u_g32;         // prefill layout: [r_p/128][din_p/64][64][4], [dout_p/128][r_p/64][64][4]
     size_t din_q, r_q;                // K of the fp4 decode layout: multiples of 128
     uint32_t *vt_q4, *u_q4;           // [r_p/64][din_q/128][64][4], [dout_p/64][r_q/128][64][4]
@@ -156,11 +156,22 @@ size_t g32_workspace(const qbk_factor *L, size_t N);
 int g32_run(const qbk_factor *L, const void *x, bool xf32, size_t N, void *y, bool ybf16, void *ws,
             hipStream_t s);
 
-// apply's fp32 serving on the device (factor.hip): the reference's row
-// bitplanes formed once, then one token's f64 product (scratch: din + r + dout
-// doubles).
-int factor_rows_ready(const qbk_factor *L, hipStream_t s);
-int factor_apply_f64_dev(qbk_ctx *ctx, const qbk_factor *L, const float *x, float *y, double *scratch,
-                         hipStream_t s);
+// serve64.hip: apply's fp32 serving of one token for up to F64_MAXL layers
+// (a group sharing an input, or one), in two launches after z.  The layers'
+// signs must be formed (factor_f64_ready, once a layer).  scratch holds
+// factor_f64_scratch doubles: per layer z then t, each in f64_pos order and
+// zero past its valid length to a multiple of 128.  factor_f64_run forms z
+// from x; factor_f64_staged runs from a z that a caller's kernel has written
+// at factor_f64_z (resid, or null, is added to every y).
+#define F64_MAXL 3
+__host__ __device__ inline uint32_t f64_pos(uint32_t k) {  // pairs k, k + 4 side by side: a 16-byte load a lane group
+    return (k & ~7u) | ((k & 3u) << 1) | ((k >> 2) & 1u);
+}
+int factor_f64_ready(const qbk_factor *L, hipStream_t s);
+size_t factor_f64_scratch(const qbk_factor *const *L, int n);
+double *factor_f64_z(const qbk_factor *const *L, int i, double *scratch);
+int factor_f64_staged(const qbk_factor *const *L, int n, float *const *y, const float *resid, double *scratch,
+                      hipStream_t s);
+int factor_f64_run(const qbk_factor *const *L, int n, const float *x, float *const *y, double *scratch, hipStream_t s);
 
 }  // namespace qbk
