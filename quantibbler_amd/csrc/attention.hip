@@ -185,6 +185,30 @@ __device__ __forceinline__ float att_sum4(float v) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// The reference r that a query's p = exp(s - r) share: n ln 2 for an integer
+// n (in two parts: the high one has 12 trailing zero bits, so n times it is
+// exact), the least at or above the running max.  Moving it scales by a power
+// of two, exactly, so running sums and the merge of the waves add no rounding
+// (with r the max itself each wave's factor carried an exp's error into the
+// result).  Past |max| = 4096 (n out of the exact range), and at infinities, r
+// is the max and n is infinite.
+struct AttRef {
+    float n, hi, lo;
+};
+__device__ __forceinline__ AttRef att_ref(float m) {
+    if (fabsf(m) < 4096.0f) {
+        const float n = ceilf(m * 1.44269504088896341f);
+        return AttRef{n, n * 0.693145751953125f, n * 1.428606765330187045e-06f};
+    }
+    return AttRef{INFINITY, m, 0.0f};
+}
+// exp(a - b), the factor of sums held at a on b; 0 where a holds none
+__device__ __forceinline__ float att_rescale(const AttRef &a, const AttRef &b) {
+    if (a.hi == -INFINITY) return 0.0f;
+    if (a.n < INFINITY && b.n < INFINITY) return ldexpf(1.0f, (int)(a.n - b.n));
+    return expf((a.hi - b.hi) + (a.lo - b.lo));
+}
+
 // One tile's part of O for 16 queries, key by key: keys a query does not see
 // add nothing, whatever their values.  p of key 16 kt + 4 G + i is in lane
 // (col, G).
@@ -221,7 +245,8 @@ __device__ __forceinline__ void att_tile_masked(const float *vb, size_t v_tok, u
 template <int DT, int NH, int QW>
 __global__ void __launch_bounds__(64 * ATT_WAVES, 2) att_tile(AttArgs a) {
     constexpr int KT = ATT_TILE_K / 16, KW = ATT_WAVES / QW;
-    __shared__ float ml[2][ATT_WAVES][16];
+    __shared__ AttRef refs[ATT_WAVES][16];
+    __shared__ float ls[ATT_WAVES][16];
     __shared__ __attribute__((aligned(16))) float ob[ATT_WAVES][16][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, G = lane >> 4, qw = wave % QW, kw = wave / QW;
@@ -253,6 +278,7 @@ __global__ void __launch_bounds__(64 * ATT_WAVES, 2) att_tile(AttArgs a) {
     }
     att_f32x4_t o[NH][4];
     float m = -INFINITY, l = 0.0f;
+    AttRef ref = att_ref(m);
 #pragma unroll
     for (int hh = 0; hh < NH; hh++)
 #pragma unroll
@@ -343,19 +369,21 @@ __global__ void __launch_bounds__(64 * ATT_WAVES, 2) att_tile(AttArgs a) {
 #pragma unroll
         for (int e = 0; e < 4 * KT; e++) cmax = fmaxf(cmax, p[e]);
         const float mn = fmaxf(m, att_max4(cmax));
-        if (__any(mn != m)) {  // some query's max moved
-            const float alpha = m == -INFINITY ? 0.0f : expf(m - mn);
+        if (__any(mn > m)) {  // some query's max moved
+            const AttRef to = mn > m ? att_ref(mn) : ref;
+            const float alpha = att_rescale(ref, to);
             l *= alpha;
 #pragma unroll
             for (int hh = 0; hh < NH; hh++)
 #pragma unroll
                 for (int j = 0; j < 4; j++) o[hh][j] *= alpha;
             m = mn;
+            ref = to;
         }
         float part = 0.0f;
 #pragma unroll
         for (int e = 0; e < 4 * KT; e++) {
-            const float x = expf(p[e] - mn);
+            const float x = expf((p[e] - ref.hi) - ref.lo);
             p[e] = p[e] == -INFINITY ? 0.0f : x;
             part += p[e];
         }
@@ -400,20 +428,24 @@ __global__ void __launch_bounds__(64 * ATT_WAVES, 2) att_tile(AttArgs a) {
         load_k(j0);
         tile(j0, 0, std::true_type{});
     }
-    // merge the waves: every wave's output and sum on the largest max
-    const float ls = att_sum4(l);
+    // merge the waves: every wave's output and sum on the largest reference
+    const float lsum = att_sum4(l);
     if (G == 0) {
-        ml[0][wave][col] = m;
-        ml[1][wave][col] = ls;
+        refs[wave][col] = ref;
+        ls[wave][col] = lsum;
     }
     __syncthreads();
-    float f;
-    {
-        float M = -INFINITY;
+    // the largest reference of query q of the workgroup's query tile t
+    auto largest = [&](int t, int q) {
+        AttRef r = refs[t][q];
 #pragma unroll
-        for (int w = 0; w < KW; w++) M = fmaxf(M, ml[0][w * QW + qw][col]);
-        f = m == -INFINITY ? 0.0f : expf(m - M);
-    }
+        for (int w = 1; w < KW; w++) {
+            const AttRef x = refs[w * QW + t][q];
+            if (x.hi > r.hi) r = x;
+        }
+        return r;
+    };
+    const float f = att_rescale(ref, largest(qw, col));
 #pragma unroll
     for (int hh = 0; hh < NH; hh++) {
         if (hh) __syncthreads();  // the first half's sums are read
@@ -429,13 +461,11 @@ __global__ void __launch_bounds__(64 * ATT_WAVES, 2) att_tile(AttArgs a) {
             const int t = x / 1024, q = x / 64 % 16, c = x % 64;
             const uint32_t i = qg + 16 * t + q;
             if (i >= Sq || 64u * hh + c >= dv) continue;
-            float M = -INFINITY, L = 0.0f, sum = 0.0f;
-#pragma unroll
-            for (int w = 0; w < KW; w++) M = fmaxf(M, ml[0][w * QW + t][q]);
+            const AttRef M = largest(t, q);
+            float L = 0.0f, sum = 0.0f;
 #pragma unroll
             for (int w = 0; w < KW; w++) {
-                const float mw = ml[0][w * QW + t][q];
-                L += ml[1][w * QW + t][q] * (mw == -INFINITY ? 0.0f : expf(mw - M));
+                L += ls[w * QW + t][q] * att_rescale(refs[w * QW + t][q], M);
                 sum += ob[w * QW + t][q][c];
             }
             a.out[((size_t)bh * a.Sq + i) * a.dv + 64 * hh + c] = sum / L;
