@@ -4,6 +4,7 @@
 // argmax (sampler.rs:4-15).  Rows are independent, so each op is one
 // workgroup per row over rows laid out contiguously.
 #include <math.h>
+#include <string.h>
 
 #include "qbk_internal.h"
 
@@ -16,14 +17,32 @@ namespace qbk {
 // out[r] = table[tokens[r]] (f32 rows of d).  An id outside the vocabulary
 // writes a row of NaN: a device-side id cannot raise the reference's error
 // synchronously, so it poisons the row instead (the host form validates).
-__global__ void __launch_bounds__(TRUNK_THREADS) trunk_embed(const float *table, size_t vocab, size_t d,
-                                                            const int32_t *tokens, float *out) {
-    const size_t row = blockIdx.x;
-    const int32_t t = tokens[row];
+__device__ __forceinline__ void trunk_embed_row(const float *table, size_t vocab, size_t d, int32_t t, float *dst) {
     const bool ok = t >= 0 && (size_t)t < vocab;
     const float *src = table + (ok ? (size_t)t : 0) * d;
-    float *dst = out + row * d;
-    for (size_t i = threadIdx.x; i < d; i += TRUNK_THREADS) dst[i] = ok ? src[i] : __builtin_nanf("");
+    for (size_t i = (size_t)blockIdx.y * TRUNK_THREADS + threadIdx.x; i < d; i += (size_t)gridDim.y * TRUNK_THREADS)
+        dst[i] = ok ? src[i] : __builtin_nanf("");
+}
+__global__ void __launch_bounds__(TRUNK_THREADS) trunk_embed(const float *table, size_t vocab, size_t d,
+                                                            const int32_t *tokens, float *out) {
+    trunk_embed_row(table, vocab, d, tokens[blockIdx.x], out + (size_t)blockIdx.x * d);
+}
+
+// Host ids as a kernel argument: no device buffer, copy or free a call (those
+// cost a decode step's call about 20 us of host and device time).
+#define TRUNK_ARG_IDS 256
+struct TrunkIds {
+    int32_t id[TRUNK_ARG_IDS];
+};
+__global__ void __launch_bounds__(TRUNK_THREADS) trunk_embed_ids(const float *table, size_t vocab, size_t d,
+                                                                TrunkIds ids, float *out) {
+    trunk_embed_row(table, vocab, d, ids.id[blockIdx.x], out + (size_t)blockIdx.x * d);
+}
+
+// Workgroups a row: the row's loads in flight over more CUs than one.
+static unsigned trunk_embed_split(size_t d) {
+    const size_t n = div_ceil(d, 4 * TRUNK_THREADS);
+    return (unsigned)(n < 16 ? n : 16);
 }
 
 // norm_apply at bf16 serving (engine/mod.rs:837-852 over rms_norm_into,
@@ -38,10 +57,35 @@ __global__ void __launch_bounds__(TRUNK_THREADS) trunk_rms_norm(const float *x, 
     __shared__ float red[TRUNK_THREADS / 64];
     const float *xr = x + (size_t)blockIdx.x * d;
     float *orow = out + (size_t)blockIdx.x * d;
+    // Rows of up to TRUNK_THREADS * PER elements: every load issued before
+    // the first sum and the row read once (one at a time, one row of 4096
+    // took 11 us); the sums run in the same order either way.
+    constexpr int PER = 32;
+    const bool held = d <= (size_t)TRUNK_THREADS * PER;
+    float xv[PER], wv[PER];
     float ss = 0.0f;
-    for (size_t i = threadIdx.x; i < d; i += TRUNK_THREADS) {
-        const float b = F32 ? xr[i] : bf16_to_f32(f32_to_bf16(xr[i]));
-        ss += b * b;
+    if (held) {
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const size_t i = threadIdx.x + (size_t)k * TRUNK_THREADS, c = i < d ? i : 0;
+            if ((size_t)k * TRUNK_THREADS < d) {
+                xv[k] = xr[c];
+                wv[k] = w[c];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const size_t i = threadIdx.x + (size_t)k * TRUNK_THREADS;
+            if (i < d) {
+                xv[k] = F32 ? xv[k] : bf16_to_f32(f32_to_bf16(xv[k]));
+                ss += xv[k] * xv[k];
+            }
+        }
+    } else {
+        for (size_t i = threadIdx.x; i < d; i += TRUNK_THREADS) {
+            const float b = F32 ? xr[i] : bf16_to_f32(f32_to_bf16(xr[i]));
+            ss += b * b;
+        }
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
@@ -51,6 +95,14 @@ __global__ void __launch_bounds__(TRUNK_THREADS) trunk_rms_norm(const float *x, 
 #pragma unroll
     for (int i = 0; i < TRUNK_THREADS / 64; i++) tot += red[i];
     const float inv = 1.0f / sqrtf(tot / (float)d + eps);
+    if (held) {
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const size_t i = threadIdx.x + (size_t)k * TRUNK_THREADS;
+            if (i < d) orow[i] = F32 ? xv[k] * inv * wv[k] : bf16_to_f32(f32_to_bf16(xv[k] * inv * wv[k]));
+        }
+        return;
+    }
     for (size_t i = threadIdx.x; i < d; i += TRUNK_THREADS) {
         const float b = F32 ? xr[i] : bf16_to_f32(f32_to_bf16(xr[i]));
         orow[i] = F32 ? b * inv * w[i] : bf16_to_f32(f32_to_bf16(b * inv * w[i]));
@@ -146,13 +198,25 @@ int qbk_embed(qbk_ctx *ctx, const float *table, size_t vocab, size_t d_model, co
     if (n == 0 || d_model == 0) return QBK_OK;
     if ((rc = bind(ctx))) return rc;
     hipStream_t s = (hipStream_t)stream;
+    // a few hundred ids travel in the launches themselves (a decode step's, a
+    // short prompt's), a longer list through a buffer
     DevBuf ids;
-    if ((rc = ids.alloc(n * 4))) return rc;
-    QBK_HIP(hipMemcpy(ids.p, tokens_host, n * 4, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(trunk_embed, dim3((unsigned)n), dim3(TRUNK_THREADS), 0, s, table, vocab, d_model,
-                       (const int32_t *)ids.p, out);
+    if (n <= 4 * TRUNK_ARG_IDS) {
+        for (size_t i0 = 0; i0 < n; i0 += TRUNK_ARG_IDS) {
+            const size_t c = n - i0 < TRUNK_ARG_IDS ? n - i0 : TRUNK_ARG_IDS;
+            TrunkIds a;
+            memcpy(a.id, tokens_host + i0, c * 4);
+            hipLaunchKernelGGL(trunk_embed_ids, dim3((unsigned)c, trunk_embed_split(d_model)), dim3(TRUNK_THREADS), 0, s,
+                               table, vocab, d_model, a, out + i0 * d_model);
+        }
+    } else {
+        if ((rc = ids.alloc(n * 4))) return rc;
+        QBK_HIP(hipMemcpy(ids.p, tokens_host, n * 4, hipMemcpyHostToDevice));
+        hipLaunchKernelGGL(trunk_embed, dim3((unsigned)n, trunk_embed_split(d_model)), dim3(TRUNK_THREADS), 0, s, table,
+                           vocab, d_model, (const int32_t *)ids.p, out);
+    }
     QBK_HIP(hipGetLastError());
-    QBK_HIP(hipStreamSynchronize(s));  // the ids buffer is freed on return
+    QBK_HIP(hipStreamSynchronize(s));  // the rows are written when this returns
     return QBK_OK;
 }
 
@@ -162,8 +226,8 @@ int qbk_embed_dev(qbk_ctx *ctx, const float *table, size_t vocab, size_t d_model
     if (!table || !tokens || !out) return fail(QBK_ERR_VALIDATION, "null argument");
     if (n == 0 || d_model == 0) return QBK_OK;
     if ((rc = bind(ctx))) return rc;
-    hipLaunchKernelGGL(trunk_embed, dim3((unsigned)n), dim3(TRUNK_THREADS), 0, (hipStream_t)stream, table, vocab,
-                       d_model, tokens, out);
+    hipLaunchKernelGGL(trunk_embed, dim3((unsigned)n, trunk_embed_split(d_model)), dim3(TRUNK_THREADS), 0,
+                       (hipStream_t)stream, table, vocab, d_model, tokens, out);
     QBK_HIP(hipGetLastError());
     return QBK_OK;
 }
