@@ -427,14 +427,77 @@ __global__ void __launch_bounds__(NT) blkp_norm(const float *__restrict__ a, con
     }
 }
 
+// blkp_norm of many rows (a prefill's) of d <= 8192, d a multiple of 4 and
+// 16-byte aligned: a row a workgroup in 16-byte loads and stores, all of its
+// loads issued at once.  HBM-bound: 2048 rows of 4096, 4-byte accesses ->
+// these, 21 -> 11 us without a residual (50 MB), 41 -> 20 us with one
+// (117 MB).
+template <bool RES>
+__global__ void __launch_bounds__(256) blkp_norm4(const float *__restrict__ a, const float *__restrict__ r,
+                                                  float *__restrict__ hout, const float *__restrict__ w, float eps,
+                                                  uint16_t *__restrict__ x, uint32_t d) {
+    constexpr int NE = 8;  // 256 x 8 16-byte pieces
+    __shared__ float red[4];
+    const size_t off = (size_t)blockIdx.x * d;
+    const uint32_t tid = threadIdx.x, nq = d / 4;
+    const float4 *a4 = (const float4 *)(a + off), *r4 = (const float4 *)(r + off), *w4 = (const float4 *)w;
+    float4 v[NE], wv[NE];
+#pragma unroll
+    for (int k = 0; k < NE; k++)
+        if (256u * k < nq) {  // uniform
+            const uint32_t i = tid + 256 * k, c = i < nq ? i : nq - 1;
+            v[k] = a4[c];
+            wv[k] = w4[c];
+            if constexpr (RES) {
+                const float4 q = r4[c];
+                v[k] = make_float4(v[k].x + q.x, v[k].y + q.y, v[k].z + q.z, v[k].w + q.w);
+            }
+        }
+    float ss = 0.0f;
+#pragma unroll
+    for (int k = 0; k < NE; k++)
+        if (tid + 256 * k < nq) {
+            if constexpr (RES) ((float4 *)(hout + off))[tid + 256 * k] = v[k];
+            float *e = &v[k].x;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                e[j] = __uint_as_float((uint32_t)blkd_bf16(e[j]) << 16);
+                ss += e[j] * e[j];
+            }
+        }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
+    if ((tid & 63) == 0) red[tid >> 6] = ss;
+    __syncthreads();
+    const float tot = (red[0] + red[1]) + (red[2] + red[3]);
+    const float inv = 1.0f / sqrtf(tot / (float)d + eps);
+#pragma unroll
+    for (int k = 0; k < NE; k++)
+        if (tid + 256 * k < nq) {
+            const float *e = &v[k].x, *we = &wv[k].x;
+            uint16_t o[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) o[j] = blkd_bf16(e[j] * inv * we[j]);
+            ((uint2 *)(x + off))[tid + 256 * k] =
+                make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
+        }
+}
+
 // blkp_norm over n rows: 1024 threads a row for a few rows (a batched decode
-// step: the row's latency is the step's), 256 for many (a prefill).
+// step: the row's latency is the step's), 256 for many (a prefill), in
+// 16-byte accesses where rows allow them (r and hout go together there).
 static void blkp_norm_launch(size_t n, const float *a, const float *r, float *hout, const float *w, float eps,
                              uint16_t *x, int d, int nrep, hipStream_t s) {
+    const uintptr_t p = (uintptr_t)a | (uintptr_t)r | (uintptr_t)hout | (uintptr_t)w | (uintptr_t)x;
     if (n <= 64)
         hipLaunchKernelGGL(blkp_norm<BLKD_NORM_THREADS>, dim3((unsigned)n), dim3(BLKD_NORM_THREADS), 0, s, a, r,
                            hout, w, eps, x, d, nrep);
-    else
+    else if (nrep == 1 && d % 4 == 0 && d <= 8192 && p % 16 == 0 && !r == !hout) {
+        if (r)
+            hipLaunchKernelGGL(blkp_norm4<true>, dim3((unsigned)n), dim3(256), 0, s, a, r, hout, w, eps, x, (uint32_t)d);
+        else
+            hipLaunchKernelGGL(blkp_norm4<false>, dim3((unsigned)n), dim3(256), 0, s, a, r, hout, w, eps, x, (uint32_t)d);
+    } else
         hipLaunchKernelGGL(blkp_norm<256>, dim3((unsigned)n), dim3(256), 0, s, a, r, hout, w, eps, x, d, nrep);
 }
 
@@ -502,27 +565,6 @@ __global__ void blkp_swiglu(const float *g, const float *u, float *hid, size_t c
         const float gv = g[i], uv = u[i];
         hid[i] = gv * uv / (1.0f + expf(0.0f - gv));
     }
-}
-
-// blkp_swiglu followed by the down projection's z = bf16(s2 hid) (the
-// GEMM's f32-x conversion, the same f32 product and rounding), written as
-// bf16: the GEMM then reads it at s2 = 1, where bf16(1 * z) = z.  Half the
-// bytes of the f32 hidden row on both sides.  Four elements a thread (ffn a
-// multiple of 4).
-__global__ void blkp_swiglu_z(const float *g, const float *u, const float *s2, uint16_t *z, size_t count,
-                              uint32_t ffn) {
-    const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-    if (i >= count) return;
-    const float4 gv = *(const float4 *)(g + i), uv = *(const float4 *)(u + i);
-    const float4 sv = *(const float4 *)(s2 + i % ffn);
-    const float ga[4] = {gv.x, gv.y, gv.z, gv.w}, ua[4] = {uv.x, uv.y, uv.z, uv.w}, sa[4] = {sv.x, sv.y, sv.z, sv.w};
-    uint16_t o[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const float hid = ga[e] * ua[e] / (1.0f + expf(0.0f - ga[e]));
-        o[e] = f32_to_bf16(sa[e] * hid);
-    }
-    *(uint2 *)(z + i) = make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
 }
 
 __global__ void blkp_add(const float *a, const float *b, float *out, size_t count) {
@@ -1142,17 +1184,16 @@ int qbk_block_prefill_seq_dev(qbk_ctx *ctx, qbk_block *B, size_t seq, float *h, 
     if ((rc = blkp_proj(B->o, n, arow, false, oo, ws, s))) return rc;
     blkp_norm_launch(n, oo, h, h1, B->w_post, B->eps, x, d, 1, s);
     QBK_HIP(hipGetLastError());
-    if ((rc = blkp_proj(B->lay[4], n, x, false, g, ws, s)) || (rc = blkp_proj(B->lay[5], n, x, false, u, ws, s)))
-        return rc;
-    if (n > Q4_MAXB && q4g_use(B->down, n) && B->ffn % 4 == 0) {
-        // SwiGLU writes the down projection's z in bf16 (read at s2 = 1), and
+    if ((rc = blkp_proj(B->lay[4], n, x, false, g, ws, s))) return rc;
+    if (n > Q4_MAXB && q4g_use(B->lay[5], n) && q4g_use(B->down, n) && B->ffn % 4 == 0) {
+        // the up projection's epilogue forms SwiGLU and from it the down
+        // projection's z in bf16 (read at s2 = 1): u never goes to memory;
         // h = down + h1, the residual added in the GEMM's epilogue
         uint16_t *z = (uint16_t *)(w + P.o_z);
-        hipLaunchKernelGGL(blkp_swiglu_z, dim3((unsigned)div_ceil(nf / 4, 256)), dim3(256), 0, s, g, u,
-                           B->down->s2, z, nf, (uint32_t)B->ffn);
-        QBK_HIP(hipGetLastError());
-        if ((rc = q4g_run(B->down, z, false, n, h, false, (uint16_t *)ws, s, h1, B->ones_ffn))) return rc;
+        if ((rc = q4g_run(B->lay[5], x, false, n, z, true, nullptr, s, nullptr, nullptr, g, B->down->s2))) return rc;
+        if ((rc = q4g_run(B->down, z, false, n, h, false, nullptr, s, h1, B->ones_ffn))) return rc;
     } else {
+        if ((rc = blkp_proj(B->lay[5], n, x, false, u, ws, s))) return rc;
         hipLaunchKernelGGL(blkp_swiglu, dim3((unsigned)div_ceil(nf, 256)), dim3(256), 0, s, g, u, g, nf);
         QBK_HIP(hipGetLastError());
         if ((rc = blkp_proj(B->down, n, g, true, oo, ws, s))) return rc;
