@@ -558,6 +558,88 @@ __global__ void __launch_bounds__(256) blkp_qk_rope(const float *q, const float 
     }
 }
 
+// blkp_qk_rope at a head dim of 128 and 16-byte aligned operands: 16 lanes a
+// head, each four channels of either half in 16-byte loads (the bf16 rows in
+// 8-byte stores), every load issued at once; the v heads are units of their
+// own.  The squares' sum takes blkp_qk_rope's tree -- channel j
+// with j ^ 32, ^ 16, .. ^ 1, across lanes and then within -- so all values are
+// its, bit for bit.  HBM-bound: 2048 tokens of 32/8 heads x 128 (92 MB),
+// 4-byte accesses by a wave a head -> these, 27 -> 18 us, the copy rate.
+__global__ void __launch_bounds__(256) blkp_qk_rope4(const float *__restrict__ q, const float *__restrict__ k,
+                                                     const float *__restrict__ v, const float2 *__restrict__ rope,
+                                                     const float *__restrict__ wq, const float *__restrict__ wk,
+                                                     float eps, float *__restrict__ kc, float *__restrict__ vc,
+                                                     uint16_t *__restrict__ qb, uint16_t *__restrict__ kb,
+                                                     uint16_t *__restrict__ vb, int H, int Hk, int n) {
+    constexpr int HD = 128, L = 16, half = 64;
+    const int heads = H + 2 * Hk, head = (int)blockIdx.x * (256 / L) + (int)threadIdx.x / L, t = blockIdx.y;
+    if (head >= heads) return;  // whole heads' lanes; no barrier follows
+    const int j = 4 * ((int)threadIdx.x & (L - 1));  // channels j .. j + 3 and half + j ..
+    const bool is_q = head < H, is_v = head >= H + Hk;
+    const int hh = is_q ? head : is_v ? head - H - Hk : head - H;
+    const size_t row = ((size_t)t * (is_q ? H : Hk) + hh) * HD, orow = ((size_t)hh * n + t) * HD;
+    const float *src = (is_q ? q : is_v ? v : k) + row;
+    const float4 xa = *(const float4 *)(src + j), xb = *(const float4 *)(src + half + j);
+    float a[4] = {xa.x, xa.y, xa.z, xa.w}, b[4] = {xb.x, xb.y, xb.z, xb.w};
+    if (!is_v) {
+        const float4 *cs = (const float4 *)(rope + (size_t)t * half + j);
+        const float4 c0 = cs[0], c1 = cs[1];
+        const float co[4] = {c0.x, c0.z, c1.x, c1.z}, si[4] = {c0.y, c0.w, c1.y, c1.w};
+        const float *w = is_q ? wq : wk;
+        if (w) {
+            const float4 w0 = *(const float4 *)(w + j), w1 = *(const float4 *)(w + half + j);
+            const float wa[4] = {w0.x, w0.y, w0.z, w0.w}, wb[4] = {w1.x, w1.y, w1.z, w1.w};
+            float ss[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                a[e] = bf16_to_f32(f32_to_bf16(a[e]));
+                b[e] = bf16_to_f32(f32_to_bf16(b[e]));
+                ss[e] = a[e] * a[e] + b[e] * b[e];  // bf16 squares are exact
+#pragma unroll
+                for (int o = L / 2; o >= 1; o >>= 1) ss[e] += __shfl_xor(ss[e], o, 64);
+            }
+            const float inv = 1.0f / sqrtf(((ss[0] + ss[2]) + (ss[1] + ss[3])) / (float)HD + eps);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                a[e] = bf16_to_f32(f32_to_bf16(a[e] * inv * wa[e]));
+                b[e] = bf16_to_f32(f32_to_bf16(b[e] * inv * wb[e]));
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float ra = a[e] * co[e] - b[e] * si[e], rb = b[e] * co[e] + a[e] * si[e];
+            a[e] = ra;
+            b[e] = rb;
+        }
+    }
+    uint16_t *ob = (is_q ? qb : is_v ? vb : kb) + orow;
+    const auto pk = [](const float *x) {
+        return make_uint2((uint32_t)f32_to_bf16(x[0]) | ((uint32_t)f32_to_bf16(x[1]) << 16),
+                          (uint32_t)f32_to_bf16(x[2]) | ((uint32_t)f32_to_bf16(x[3]) << 16));
+    };
+    *(uint2 *)(ob + j) = pk(a);
+    *(uint2 *)(ob + half + j) = pk(b);
+    if (!is_q) {
+        float *crow = (is_v ? vc : kc) + row;
+        *(float4 *)(crow + j) = make_float4(a[0], a[1], a[2], a[3]);
+        *(float4 *)(crow + half + j) = make_float4(b[0], b[1], b[2], b[3]);
+    }
+}
+
+static void blkp_qk_rope_launch(const float *q, const float *k, const float *v, const float2 *rope, const float *wq,
+                                const float *wk, float eps, float *kc, float *vc, uint16_t *qb, uint16_t *kb,
+                                uint16_t *vb, int H, int Hk, int hd, size_t n, hipStream_t s) {
+    const uintptr_t p = (uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)rope | (uintptr_t)wq | (uintptr_t)wk |
+                        (uintptr_t)kc | (uintptr_t)vc | (uintptr_t)qb | (uintptr_t)kb | (uintptr_t)vb;
+    const int heads = H + 2 * Hk;
+    if (hd == 128 && p % 16 == 0)
+        hipLaunchKernelGGL(blkp_qk_rope4, dim3((heads + 15) / 16, (unsigned)n), dim3(256), 0, s, q, k, v, rope, wq,
+                           wk, eps, kc, vc, qb, kb, vb, H, Hk, (int)n);
+    else
+        hipLaunchKernelGGL(blkp_qk_rope, dim3((H + Hk + 3) / 4, (unsigned)n), dim3(256), 0, s, q, k, v, rope, wq, wk,
+                           eps, kc, vc, qb, kb, vb, H, Hk, hd, (int)n);
+}
+
 // hidden = g u / (1 + exp(-g)), elementwise over n rows of ffn
 __global__ void blkp_swiglu(const float *g, const float *u, float *hid, size_t count) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1173,8 +1255,8 @@ int qbk_block_prefill_seq_dev(qbk_ctx *ctx, qbk_block *B, size_t seq, float *h, 
         (rc = blkp_proj(B->lay[2], n, x, false, v, ws, s)))
         return rc;
     const size_t kvs = B->cap * B->Hk * B->hd;  // one sequence's cache floats
-    hipLaunchKernelGGL(blkp_qk_rope, dim3((H + Hk + 3) / 4, (unsigned)n), dim3(256), 0, s, q, k, v, B->rope, B->w_q, B->w_k,
-                       B->eps, B->kc + seq * kvs, B->vc + seq * kvs, qb, kb, vb, H, Hk, hd, (int)n);
+    blkp_qk_rope_launch(q, k, v, B->rope, B->w_q, B->w_k, B->eps, B->kc + seq * kvs, B->vc + seq * kvs, qb, kb, vb, H,
+                        Hk, hd, n, s);
     QBK_HIP(hipGetLastError());
     // causal block-scaled SageAttention over the n tokens
     const qbk_attn_shape sh{1, B->H, B->Hk, n, n, B->hd, B->hd};
