@@ -427,60 +427,81 @@ __global__ void __launch_bounds__(NT) blkp_norm(const float *__restrict__ a, con
     }
 }
 
-// blkp_norm of many rows (a prefill's) of d <= 8192, d a multiple of 4 and
-// 16-byte aligned: a row a workgroup in 16-byte loads and stores, all of its
-// loads issued at once.  HBM-bound: 2048 rows of 4096, 4-byte accesses ->
-// these, 21 -> 11 us without a residual (50 MB), 41 -> 20 us with one
-// (117 MB).
-template <bool RES>
+// blkp_norm<256> of many rows (a prefill's) of d <= 8192, d a multiple of 4
+// and 16-byte aligned: a row a workgroup in 16-byte loads and stores, all of
+// its loads issued at once.  The bf16 row passes through LDS, from which
+// thread t sums channels t, t + 256, .. in turn, as blkp_norm<256>'s does:
+// every value is that kernel's, bit for bit.  HBM-bound: 2048 rows of 4096,
+// 4-byte accesses -> these, 21 -> 11 us without a residual (50 MB), 41 -> 20 us
+// with one (117 MB).  (A wave a row, whose lanes hold such sums whole, takes
+// the same at 2048 rows and 4 us more a launch at 65 to 777.)
+// NE: 16-byte pieces a thread, 1024 NE >= d.
+template <bool RES, int NE>
 __global__ void __launch_bounds__(256) blkp_norm4(const float *__restrict__ a, const float *__restrict__ r,
                                                   float *__restrict__ hout, const float *__restrict__ w, float eps,
                                                   uint16_t *__restrict__ x, uint32_t d) {
-    constexpr int NE = 8;  // 256 x 8 16-byte pieces
     __shared__ float red[4];
+    __shared__ uint2 xs[256 * NE];  // the row in bf16, zero past d
     const size_t off = (size_t)blockIdx.x * d;
     const uint32_t tid = threadIdx.x, nq = d / 4;
     const float4 *a4 = (const float4 *)(a + off), *r4 = (const float4 *)(r + off), *w4 = (const float4 *)w;
-    float4 v[NE], wv[NE];
+    float4 v[NE], q[NE], wv[NE];
 #pragma unroll
-    for (int k = 0; k < NE; k++)
-        if (256u * k < nq) {  // uniform
-            const uint32_t i = tid + 256 * k, c = i < nq ? i : nq - 1;
-            v[k] = a4[c];
-            wv[k] = w4[c];
-            if constexpr (RES) {
-                const float4 q = r4[c];
-                v[k] = make_float4(v[k].x + q.x, v[k].y + q.y, v[k].z + q.z, v[k].w + q.w);
-            }
-        }
+    for (int k = 0; k < NE; k++) {
+        const uint32_t i = tid + 256 * k, c = i < nq ? i : nq - 1;
+        v[k] = a4[c];
+        if constexpr (RES) q[k] = r4[c];
+        wv[k] = w4[c];
+    }
+    uint2 bv[NE];
+#pragma unroll
+    for (int k = 0; k < NE; k++) {
+        if constexpr (RES) v[k] = make_float4(v[k].x + q[k].x, v[k].y + q[k].y, v[k].z + q[k].z, v[k].w + q[k].w);
+        const float *e = &v[k].x;
+        bv[k] = make_uint2((uint32_t)blkd_bf16(e[0]) | ((uint32_t)blkd_bf16(e[1]) << 16),
+                           (uint32_t)blkd_bf16(e[2]) | ((uint32_t)blkd_bf16(e[3]) << 16));
+        xs[tid + 256 * k] = tid + 256 * k < nq ? bv[k] : make_uint2(0, 0);
+    }
+    __syncthreads();
     float ss = 0.0f;
 #pragma unroll
-    for (int k = 0; k < NE; k++)
-        if (tid + 256 * k < nq) {
-            if constexpr (RES) ((float4 *)(hout + off))[tid + 256 * k] = v[k];
-            float *e = &v[k].x;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                e[j] = __uint_as_float((uint32_t)blkd_bf16(e[j]) << 16);
-                ss += e[j] * e[j];
-            }
-        }
+    for (int k = 0; k < 4 * NE; k++) {
+        const float b = __uint_as_float((uint32_t)((const uint16_t *)xs)[tid + 256 * k] << 16);
+        ss += b * b;
+    }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
     if ((tid & 63) == 0) red[tid >> 6] = ss;
+    if constexpr (RES) {
+#pragma unroll
+        for (int k = 0; k < NE; k++)
+            if (tid + 256 * k < nq) ((float4 *)(hout + off))[tid + 256 * k] = v[k];
+    }
     __syncthreads();
-    const float tot = (red[0] + red[1]) + (red[2] + red[3]);
+    float tot = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) tot += red[i];
     const float inv = 1.0f / sqrtf(tot / (float)d + eps);
 #pragma unroll
     for (int k = 0; k < NE; k++)
         if (tid + 256 * k < nq) {
-            const float *e = &v[k].x, *we = &wv[k].x;
+            const float *we = &wv[k].x;
+            const float e[4] = {__uint_as_float(bv[k].x << 16), __uint_as_float(bv[k].x & 0xffff0000u),
+                                __uint_as_float(bv[k].y << 16), __uint_as_float(bv[k].y & 0xffff0000u)};
             uint16_t o[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) o[j] = blkd_bf16(e[j] * inv * we[j]);
             ((uint2 *)(x + off))[tid + 256 * k] =
                 make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
         }
+}
+template <int NE>
+static void blkp_norm4_launch(size_t n, const float *a, const float *r, float *hout, const float *w, float eps,
+                              uint16_t *x, uint32_t d, hipStream_t s) {
+    if (r)
+        hipLaunchKernelGGL((blkp_norm4<true, NE>), dim3((unsigned)n), dim3(256), 0, s, a, r, hout, w, eps, x, d);
+    else
+        hipLaunchKernelGGL((blkp_norm4<false, NE>), dim3((unsigned)n), dim3(256), 0, s, a, r, hout, w, eps, x, d);
 }
 
 // blkp_norm over n rows: 1024 threads a row for a few rows (a batched decode
@@ -493,10 +514,14 @@ static void blkp_norm_launch(size_t n, const float *a, const float *r, float *ho
         hipLaunchKernelGGL(blkp_norm<BLKD_NORM_THREADS>, dim3((unsigned)n), dim3(BLKD_NORM_THREADS), 0, s, a, r,
                            hout, w, eps, x, d, nrep);
     else if (nrep == 1 && d % 4 == 0 && d <= 8192 && p % 16 == 0 && !r == !hout) {
-        if (r)
-            hipLaunchKernelGGL(blkp_norm4<true>, dim3((unsigned)n), dim3(256), 0, s, a, r, hout, w, eps, x, (uint32_t)d);
+        if (d <= 1024)
+            blkp_norm4_launch<1>(n, a, r, hout, w, eps, x, (uint32_t)d, s);
+        else if (d <= 2048)
+            blkp_norm4_launch<2>(n, a, r, hout, w, eps, x, (uint32_t)d, s);
+        else if (d <= 4096)
+            blkp_norm4_launch<4>(n, a, r, hout, w, eps, x, (uint32_t)d, s);
         else
-            hipLaunchKernelGGL(blkp_norm4<false>, dim3((unsigned)n), dim3(256), 0, s, a, r, hout, w, eps, x, (uint32_t)d);
+            blkp_norm4_launch<8>(n, a, r, hout, w, eps, x, (uint32_t)d, s);
     } else
         hipLaunchKernelGGL(blkp_norm<256>, dim3((unsigned)n), dim3(256), 0, s, a, r, hout, w, eps, x, d, nrep);
 }

@@ -1,0 +1,51 @@
+"""GPU: a prompt's faster kernels against the general ones they stand in for,
+bit for bit.  A row stream h that is not 16-byte aligned takes the general
+norm (and the element-wise GEMM store), so the same prompt at an aligned and
+at an unaligned h must leave the same bits."""
+import numpy as np
+import pytest
+
+from test_gpu_block import scaled_layer
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+def make_block(orc, ctx, seed, d, ffn, H, Hk, capacity, n_seqs=1, qk_norm=False):
+    from quantibbler_amd import DecoderBlock, FactorLayer
+
+    hd = 128
+    rng = np.random.default_rng(seed)
+    shapes = [(H * hd, d, 64), (Hk * hd, d, 32), (Hk * hd, d, 32), (d, H * hd, 64), (ffn, d, 96), (ffn, d, 96),
+              (d, ffn, 96)]
+    layers = [scaled_layer(orc, rng, *s) for s in shapes]
+    devs = [FactorLayer.from_rows(ctx, L["dout"], L["din"], L["r"], L["ub"], L["vt"], L["s1"], L["s2"], L["bias"])
+            for L in layers]
+    bfv = lambda a: orc.bf16_to_f32(orc.f32_to_bf16(a.astype(np.float32)))
+    norms = [bfv(1.0 + 0.1 * rng.standard_normal(d)) for _ in range(2)]
+    heads = {k: bfv(1.0 + 0.1 * rng.standard_normal(hd)) for k in ("q_norm", "k_norm")} if qk_norm else {}
+    return DecoderBlock(ctx, devs, norms[0], norms[1], H, Hk, hd, 500000.0, 1e-5, capacity, n_seqs=n_seqs, **heads)
+
+
+def prefill(block, h, shift=0):
+    """The prompt's rows after the block, from an h that starts `shift` floats past a 256-byte boundary."""
+    n, d = h.shape
+    buf = torch.empty(n * d + shift, dtype=torch.float32, device="cuda")
+    rows = buf[shift:].view(n, d)
+    rows.copy_(torch.from_numpy(h))
+    need = block.prefill_workspace_size(n)
+    block.prefill_dev(rows, n, torch.empty(need, dtype=torch.uint8, device="cuda"), need, torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    return rows.cpu().numpy()
+
+
+@pytest.mark.parametrize("n,d", [(65, 4), (70, 252), (66, 256), (256, 260), (300, 1028), (68, 4096), (67, 4100), (65, 8192)])
+def test_norm_in_16_byte_pieces_keeps_the_sums(orc, n, d):
+    from quantibbler_amd import GpuContext
+
+    print("prompt norm bits", n, d, flush=True)
+    block = make_block(orc, GpuContext(0), n + d, d, 256, 2, 1, n)
+    h = np.random.default_rng(n * d).standard_normal((n, d)).astype(np.float32)
+    h *= np.exp(np.random.default_rng(d).standard_normal((1, d))).astype(np.float32)
+    assert prefill(block, h).tobytes() == prefill(block, h, 1).tobytes()
+    block.close()
