@@ -303,14 +303,18 @@ __device__ __forceinline__ uint32_t q4g_pair_u(uint32_t v) {
 // a lane pair's four rows are all in or all out; otherwise element by
 // element.  The two are separate kernels: one store per row tile keeps the
 // count of memory operations in flight the same on every path, which the
-// waits on the sign ring rely on.
-template <bool VECY>
+// waits on the sign ring rely on.  GATE (bf16 y and VECY only) has kernels of
+// its own for the same reason: its gate loads go out behind the ring's refill,
+// so waiting for them drains the ring, and as a branch of the plain kernels
+// they took the counts of those down with them (4096 x 4096 of rank 1024, 2048
+// tokens: 33.3 -> 33.7 us with bf16 y, 34.9 -> 36.5 with f32).
+template <bool VECY, bool GATE>
 __device__ __forceinline__ void q4g_epilogue2(const f32x4_t acc[4], const Q4GArgs &a, size_t g, const float *sb,
                                               size_t n0, int lane, bool ybf16) {
     const int col = lane & 15, G = lane >> 4, odd = col & 1;
     const size_t n = n0 + (col >> 1);
     float2 gv[4], zv[4];
-    if (VECY && a.gate) {  // the group's gate values and scales, all in flight
+    if constexpr (GATE) {  // the group's gate values and scales, all in flight
         const size_t nc = n < a.N ? n : a.N - 1;
 #pragma unroll
         for (int rt = 0; rt < 4; rt++) {
@@ -325,7 +329,7 @@ __device__ __forceinline__ void q4g_epilogue2(const f32x4_t acc[4], const Q4GArg
         const int r2 = 16 * rt + 4 * G + 2 * odd;  // this lane's first row within the group
         float y[2];
         q4g_y2(acc, rt, odd != 0, sb, r2, y);
-        if (VECY && a.gate) {
+        if constexpr (GATE) {
             const float h0 = gv[rt].x * y[0] / (1.0f + expf(0.0f - gv[rt].x));
             const float h1 = gv[rt].y * y[1] / (1.0f + expf(0.0f - gv[rt].y));
             y[0] = zv[rt].x * h0;
@@ -386,7 +390,7 @@ __device__ __forceinline__ void q4g_prio(uint32_t level) {
 // NG1: stage-1 row groups a wave accumulates (1: r_p <= 1024, 2: r_p <=
 // 2048).  Stage 1's unit: one slice of the wave's NG1 row groups (their B
 // fragment read once); stage 2's unit: one slice of a pair of row groups.
-template <bool XF32, bool YBF16, int NG1, bool VECY>
+template <bool XF32, bool YBF16, int NG1, bool VECY, bool GATE = false>
 __global__ void __launch_bounds__(64 * Q4G_WAVES) q4g_kernel(Q4GArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t q4g_lds[];
     uint8_t *xbuf = q4g_lds;                             // [2][Q4G_CH slices]
@@ -559,8 +563,8 @@ __global__ void __launch_bounds__(64 * Q4G_WAVES) q4g_kernel(Q4GArgs a) {
         __builtin_amdgcn_wave_barrier();
         Q4G_SCALES2(p + 1 < np2 ? p + 1 : p)
         const size_t g0 = (size_t)wave + Q4G_WAVES * (2 * p);
-        q4g_epilogue2<VECY>(acc2[0], a, g0, sb, n0, lane, YBF16);
-        if (two) q4g_epilogue2<VECY>(acc2[1], a, g0 + Q4G_WAVES, sb + 128, n0, lane, YBF16);
+        q4g_epilogue2<VECY, GATE>(acc2[0], a, g0, sb, n0, lane, YBF16);
+        if (two) q4g_epilogue2<VECY, GATE>(acc2[1], a, g0 + Q4G_WAVES, sb + 128, n0, lane, YBF16);
         __builtin_amdgcn_wave_barrier();
     }
 #undef Q4G_ISSUE2
@@ -571,15 +575,17 @@ __global__ void __launch_bounds__(64 * Q4G_WAVES) q4g_kernel(Q4GArgs a) {
 // host side
 // ------------------------------------------------------------------------
 
-// Every instantiation, indexed by xf32 << 3 | ybf16 << 2 | (NG1 == 2) << 1 | vecy.
+// Every instantiation, indexed by xf32 << 3 | ybf16 << 2 | (NG1 == 2) << 1 |
+// vecy; then those with a gate, 16 | (NG1 == 2).
 #define Q4G_K(XF, YB, NG, VY) (const void *)q4g_kernel<XF, YB, NG, VY>
-static const void *const q4g_kernels[16] = {
+static const void *const q4g_kernels[18] = {
     Q4G_K(false, false, 1, false), Q4G_K(false, false, 1, true), Q4G_K(false, false, 2, false),
     Q4G_K(false, false, 2, true),  Q4G_K(false, true, 1, false), Q4G_K(false, true, 1, true),
     Q4G_K(false, true, 2, false),  Q4G_K(false, true, 2, true),  Q4G_K(true, false, 1, false),
     Q4G_K(true, false, 1, true),   Q4G_K(true, false, 2, false), Q4G_K(true, false, 2, true),
     Q4G_K(true, true, 1, false),   Q4G_K(true, true, 1, true),   Q4G_K(true, true, 2, false),
-    Q4G_K(true, true, 2, true)};
+    Q4G_K(true, true, 2, true),    (const void *)q4g_kernel<false, true, 1, true, true>,
+    (const void *)q4g_kernel<false, true, 2, true, true>};
 #undef Q4G_K
 
 // x chunks, stage 2's operand, each wave's s1 / bias staging (1 KiB)
@@ -616,7 +622,7 @@ int gemm_run(const qbk_factor *L, const void *x, bool xf32, size_t N, void *y, b
 int q4g_run(const qbk_factor *L, const void *x, bool xf32, size_t N, void *y, bool ybf16, uint16_t *t_out,
             hipStream_t s, const float *resid, const float *s2, const float *gate, const float *zs2) {
     if (resid && ybf16) return fail(QBK_ERR_VALIDATION, "the GEMM adds a residual to an f32 output only");
-    if (gate && (!ybf16 || !zs2 || L->dout % 4 != 0 || (uintptr_t)y % 8 != 0 || (uintptr_t)gate % 8 != 0))
+    if (gate && (xf32 || !ybf16 || !zs2 || L->dout % 4 != 0 || (uintptr_t)y % 8 != 0 || (uintptr_t)gate % 8 != 0))
         return fail(QBK_ERR_VALIDATION, "the GEMM forms SwiGLU in bf16 rows of a multiple of 4 only");
     const uint32_t lds = q4g_lds_bytes(L);
     {
@@ -661,7 +667,7 @@ int q4g_run(const qbk_factor *L, const void *x, bool xf32, size_t N, void *y, bo
     const dim3 grid((unsigned)div_ceil(N, 8)), block(64 * Q4G_WAVES);
     // one row group a wave in stage 1 up to 16 groups (r_p <= 1024), two up to 32
     const bool two = a.n_rg1 > Q4G_WAVES;
-    const void *k = q4g_kernels[(xf32 ? 8 : 0) | (ybf16 ? 4 : 0) | (two ? 2 : 0) | (a.vec_y ? 1 : 0)];
+    const void *k = q4g_kernels[gate ? 16 + two : (xf32 ? 8 : 0) | (ybf16 ? 4 : 0) | (two ? 2 : 0) | (a.vec_y ? 1 : 0)];
     void *args[] = {&a};
     QBK_HIP(hipLaunchKernel(k, grid, block, args, lds, s));
     QBK_HIP(hipGetLastError());

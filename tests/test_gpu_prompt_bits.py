@@ -49,3 +49,38 @@ def test_norm_in_16_byte_pieces_keeps_the_sums(orc, n, d):
     h *= np.exp(np.random.default_rng(d).standard_normal((1, d))).astype(np.float32)
     assert prefill(block, h).tobytes() == prefill(block, h, 1).tobytes()
     block.close()
+
+
+@pytest.mark.parametrize("n,ffn,r", [(256, 512, 96), (261, 508, 96), (1031, 260, 40), (300, 512, 1100)])
+def test_swiglu_in_the_epilogue_is_the_separate_pass(orc, n, ffn, r):
+    """The up projection's epilogue forms SwiGLU at an ffn that is a multiple of
+    4; two more ffn rows whose gate is 0 (s1 = bias = 0) add zeros to the down
+    projection's sums and take the general kernels: f32 rows of gate and up,
+    the SwiGLU pass, the down GEMM on f32 rows, the residual's pass."""
+    from quantibbler_amd import DecoderBlock, FactorLayer, GpuContext
+
+    print("prompt swiglu bits", n, ffn, r, flush=True)
+    ctx, d, H, Hk, hd = GpuContext(0), 256, 2, 1, 128
+    rng = np.random.default_rng(n + ffn + r)
+    att = [scaled_layer(orc, rng, *s) for s in [(H * hd, d, 64), (Hk * hd, d, 32), (Hk * hd, d, 32), (d, H * hd, 64)]]
+    gate, up = scaled_layer(orc, rng, ffn + 2, d, r), scaled_layer(orc, rng, ffn + 2, d, r)
+    gate["s1"][ffn:] = gate["bias"][ffn:] = 0.0
+    vts = rng.choice([-1, 1], (r, ffn + 2)).astype(np.int8)
+    down = scaled_layer(orc, rng, d, ffn + 2, r)
+    down["vt"] = orc.pack_bits(vts)
+    h = rng.standard_normal((n, d)).astype(np.float32)
+
+    def rows(L, m):
+        return dict(L, dout=m, ub=L["ub"][:m], s1=L["s1"][:m], bias=L["bias"][:m])
+
+    outs = []
+    for f in (ffn, ffn + 2):
+        mlp = [rows(gate, f), rows(up, f),
+               dict(down, din=f, vt=orc.pack_bits(np.ascontiguousarray(vts[:, :f])), s2=down["s2"][:f])]
+        devs = [FactorLayer.from_rows(ctx, L["dout"], L["din"], L["r"], L["ub"], L["vt"], L["s1"], L["s2"], L["bias"])
+                for L in att + mlp]
+        ones = np.ones(d, np.float32)
+        block = DecoderBlock(ctx, devs, ones, ones, H, Hk, hd, 500000.0, 1e-5, n)
+        outs.append(prefill(block, h))
+        block.close()
+    assert np.isfinite(outs[0]).all() and outs[0].tobytes() == outs[1].tobytes()
