@@ -738,8 +738,8 @@ int orc_attention_sage_np_f64(const orc_attn_shape *sh, const double *q, const d
 
 /* exp(x) for the f32 reference scheme, written from the mathematics:
  * Cody & Waite (1980) reduction x = n*ln2 + r with ln2 split in two parts
- * (the high part has 12 trailing zero bits, so n*ln2_hi is exact for
- * |n| < 2^12), |r| <= ln2/2, then e^r by the degree-7 Taylor polynomial
+ * (the high part has 9 trailing zero bits, so n*ln2_hi is exact for
+ * |n| <= 2^9; here |n| <= 150), |r| <= ln2/2, then e^r by the degree-7 Taylor polynomial
  * (truncation 0.3466^8/8! < 6e-9), and the result scaled by 2^n through the
  * exponent field in two steps (so 2^n never overflows on its own).
  * The device kernel carries the same operation sequence, so the two agree

@@ -186,19 +186,22 @@ __device__ __forceinline__ float att_sum4(float v) {
 }
 
 // The reference r that a query's p = exp(s - r) share: n ln 2 for an integer
-// n (in two parts: the high one has 12 trailing zero bits, so n times it is
-// exact), the least at or above the running max.  Moving it scales by a power
-// of two, exactly, so running sums and the merge of the waves add no rounding
-// (with r the max itself each wave's factor carried an exp's error into the
-// result).  Past |max| = 4096 (n out of the exact range), and at infinities, r
-// is the max and n is infinite.
+// n, the least at or above the running max, in two parts.  Moving it scales by
+// a power of two, exactly, so running sums and the merge of the waves add no
+// rounding (with r the max itself each wave's factor carried an exp's error
+// into the result) -- as long as hi + lo is n ln 2 for every n: the high part,
+// 355 / 512, has nine significant bits, so n times it is exact to n = 2^15,
+// and n times the low part is off by 2^-23 of n 2.1e-4 at most.  (A high part
+// of fifteen bits was exact to n = 512 only: scores of 600 to 3500 then cost
+// 2e-5 to 3e-5 of the result.)  Past |max| = 4096 (n lo nears 1 there), and at
+// infinities, r is the max and n is infinite.
 struct AttRef {
     float n, hi, lo;
 };
 __device__ __forceinline__ AttRef att_ref(float m) {
     if (fabsf(m) < 4096.0f) {
         const float n = ceilf(m * 1.44269504088896341f);
-        return AttRef{n, n * 0.693145751953125f, n * 1.428606765330187045e-06f};
+        return AttRef{n, n * 0.693359375f, n * -2.12194440054690583e-4f};
     }
     return AttRef{INFINITY, m, 0.0f};
 }

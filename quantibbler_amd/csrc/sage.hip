@@ -39,8 +39,8 @@ namespace qbk {
 #pragma clang fp contract(off)
 
 // exp(x): Cody & Waite (1980) reduction x = n ln2 + r with ln2 split in two
-// (the high part has 12 trailing zero bits, so n*ln2_hi is exact), e^r by
-// the degree-7 Taylor polynomial on |r| <= ln2/2, scaled by 2^n in two
+// (the high part has 9 trailing zero bits, so n*ln2_hi is exact: |n| <= 150),
+// e^r by the degree-7 Taylor polynomial on |r| <= ln2/2, scaled by 2^n in two
 // exponent-field steps.  Written without fused multiply-add so host and
 // device agree bit for bit.
 __device__ __forceinline__ float qbk_expf(float x) {

@@ -102,3 +102,28 @@ def test_masked_and_infinite_entries_stay_where_they_belong(ctx, d):
         lim = (2 * (d / 2 + 4) * EPS * (np.abs(k[0, 0, keep]).astype(np.float64) @ np.abs(x)).max() / np.sqrt(d)
                + 64 * EPS) * np.abs(finite[0, 0, keep]).max()
         assert np.all(np.abs(got[i] - w)[check[i]] <= lim)
+
+
+@pytest.mark.parametrize("top", [3.0, 300.0, 600.0, 700.0, 1500.0, 3500.0, 4090.0, -700.0, -3500.0, 4100.0, 20000.0])
+def test_large_scores_lose_nothing(ctx, top):
+    """Scores that are f32 values exactly (one channel, a scale of 1/8), their
+    maxima spread over the key tiles and so over the waves, about `top`.
+
+    With the scores exact, a weight is off by the reference's low part (at most
+    2^-23 of 1.26, 2.6 eps, eps = 2^-24), the difference's rounding (1 eps) and
+    expf (2 eps); both sums of the quotient carry that, 11.2 eps, and the sums
+    of 1300 terms in blocks of 32 (f32 roundings of either sign) 5 eps: 16 eps
+    of max|v|.  Past 4096 the reference is the max itself and each of a wave's
+    at most 6 tiles and the merge scale by an expf (2 eps) with a rounding
+    (1 eps), in both sums: 2 x 3 x 7 eps more."""
+    rng = np.random.default_rng(int(abs(top)))
+    sq, skv, d = 20, 1300, 64
+    tile = np.arange(skv) // 32
+    s = (top - 0.7 * (tile * 5 % 13) - rng.exponential(1.0, skv)).astype(np.float32)
+    q, k = np.zeros((1, 2, sq, d), np.float32), np.zeros((1, 1, skv, d), np.float32)
+    q[..., 0], k[0, 0, :, 0] = 8.0, s
+    v = rng.choice([-1.0, 1.0], (1, 1, tile[-1] + 1, d)).astype(np.float32)[:, :, tile]  # a tile's weight shows whole
+    got = run(ctx, q, k, v, False)
+    p = np.exp(s.astype(np.float64) - float(s.max()))
+    want = p @ v[0, 0].astype(np.float64) / p.sum()
+    assert np.abs(got - want).max() <= (16 if abs(top) < 4096 else 16 + 42) * EPS * np.abs(v).max()
