@@ -268,7 +268,8 @@ __global__ void __launch_bounds__(64 * ATT_WAVES, 2) att_tile(AttArgs a) {
         return e < 0 ? 0u : e < (int64_t)Skv ? (uint32_t)e : Skv;
     };
     const uint32_t qlast = q0 + 15 < Sq ? q0 + 15 : Sq - 1;
-    const uint32_t kend_wg = q0 < Sq ? visible(qlast) : 0, kend_min = visible(q0);
+    // a wave past the last query has no keys (and only takes part in the merge)
+    const uint32_t kend_wg = q0 < Sq ? visible(qlast) : 0, kend_min = q0 < Sq ? visible(q0) : 0;
     const uint32_t iq = q0 + col < Sq ? q0 + col : Sq - 1;  // past the last: it repeats the last one, stores nothing
     const uint32_t kend = visible(iq);
     att_f32x4_t qf[DT];
