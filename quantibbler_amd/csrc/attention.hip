@@ -13,7 +13,7 @@
 // u32 index ceiling as the reference's face.
 //
 // att_tile (below) serves head dims up to 128 on the f32 matrix cores; other
-// shapes run att_exact, one workgroup per (batch, head, query row): the
+// shapes, and a few queries over few keys (att_rows_faster), run att_exact, one workgroup per (batch, head, query row): the
 // row's query in LDS, keys
 // in chunks of ATT_CHUNK -- a thread per key for the scores (dot products in
 // 16-channel partial sums), the chunk's max and sum by workgroup reductions,
@@ -492,7 +492,14 @@ static int att_tile_launch(AttArgs a, size_t B, hipStream_t st) {
     // for 1, 2, 4 tiles): 777 queries causal 124, 107, 127; 2 x 777 not causal
     // 291, 279, 255; 400 queries of d 80 over 700 keys 56, 47, 47; 64 queries
     // 44 each.
-    const int qw = div_ceil(a.Sq, 64) * B * a.H >= 400 ? 4 : div_ceil(a.Sq, 32) * B * a.H >= 150 ? 2 : 1;
+    // Tiles that hold no query leave their waves idle, so no more of them than
+    // there are queries for where the keys need the waves: 4096 single queries
+    // (us for 1 and 4 tiles) over 32 keys of d 64 67, 72; 64 keys 67, 82; 128
+    // keys 74, 121; 16 queries of 1024 heads over 32 keys 26, 22 (the merge of
+    // eight waves' outputs); 64 keys 26, 27.
+    int qw = div_ceil(a.Sq, 64) * B * a.H >= 400 ? 4 : div_ceil(a.Sq, 32) * B * a.H >= 150 ? 2 : 1;
+    if (a.Skv >= 32 + 6 * a.Sq)
+        while (qw > 1 && 8 * (size_t)qw >= a.Sq) qw /= 2;
     const size_t grid = div_ceil(a.Sq, 16 * (size_t)qw) * B * a.H;
     if (grid > 0x7FFFFFFFull) return fail(QBK_ERR_VALIDATION, "attention: too many query tiles for one launch");
     const bool small = a.d <= 64 && a.dv <= 64;

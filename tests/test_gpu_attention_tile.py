@@ -127,3 +127,18 @@ def test_large_scores_lose_nothing(ctx, top):
     p = np.exp(s.astype(np.float64) - float(s.max()))
     want = p @ v[0, 0].astype(np.float64) / p.sum()
     assert np.abs(got - want).max() <= (16 if abs(top) < 4096 else 16 + 42) * EPS * np.abs(v).max()
+
+
+@pytest.mark.parametrize("b,h,hk,sq,skv,d,dv", [
+    (26, 16, 4, 1, 38, 64, 64), (26, 16, 4, 16, 128, 64, 64), (26, 16, 4, 16, 127, 64, 64),    # one tile, one, four
+    (26, 16, 4, 17, 134, 128, 128), (26, 16, 4, 33, 230, 64, 64), (10, 16, 4, 16, 60, 80, 48),  # two, four, two
+])
+def test_query_tiles_a_workgroup(ctx, b, h, hk, sq, skv, d, dv):
+    """A few queries of many heads: as many query tiles a workgroup as the queries fill."""
+    rng = np.random.default_rng(b + sq + skv + d)
+    q = rng.standard_normal((b, h, sq, d)).astype(np.float32)
+    k = rng.standard_normal((b, hk, skv, d)).astype(np.float32)
+    v = rng.standard_normal((b, hk, skv, dv)).astype(np.float32)
+    for causal in (False, True):
+        want, bound = reference(q, k, v, causal)
+        assert np.all(np.abs(run(ctx, q, k, v, causal) - want) <= bound)
