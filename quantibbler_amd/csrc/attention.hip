@@ -485,6 +485,26 @@ static bool att_tile_fits(const AttArgs &a) {
            a.Skv <= 0x40000000u;
 }
 
+// Whether att_exact is the faster of the two for a shape that att_tile fits: a
+// few queries of many heads over few keys.  A workgroup of att_tile has a CU
+// to itself and takes 3.7 us however few keys there are (value dims past 64:
+// 7.5 us), while the rows of att_exact share one and cost by their keys.
+// Measured over 3150 shapes (heads 32 to 16384, queries 1 to 16, keys 1 to
+// 128, d 16 to 128), row kernel against tiles, us: 4096 heads of d 64, one
+// query, 1 key 18, 66; 32 keys 48, 67; 48 keys and more the tiles; two queries,
+// 16 keys 58, 71; four queries, 8 keys 82, 72; d 128, one query, 32 keys 68,
+// 124; 64 keys 162, 125.  Up to 256 heads every workgroup of att_tile has a CU
+// at once and only rows of 16 channels or fewer are better off by themselves.
+// (Heads: batches times heads.)
+static bool att_rows_faster(const AttArgs &a, size_t B) {
+    if (a.Sq > 16 || a.Skv > 64) return false;
+    const size_t BH = B * a.H, w = (a.d + a.dv) / 2;
+    const bool small = a.d <= 64 && a.dv <= 64;
+    if (BH <= 256) return w <= 16 && a.Skv <= 8 && BH * a.Sq <= 1024;
+    if (BH < 768 && a.Skv * w > (small ? 512 : 2048)) return false;
+    return a.Sq * (20 + w + a.Skv * (2 + w / 16)) <= (small ? 360 : 730);
+}
+
 static int att_tile_launch(AttArgs a, size_t B, hipStream_t st) {
     a.BH = (uint32_t)(B * a.H);
     // More query tiles a workgroup share each key's and value's way through
@@ -564,7 +584,7 @@ static int launch_exact(const qbk_attn_shape *s, const float *q, const float *k,
               s->seq_kv * s->val_dim};
     const size_t rows = s->batch * s->n_heads * s->seq_q;
     if (rows > 0x7FFFFFFFull) return fail(QBK_ERR_VALIDATION, "attention: too many query rows for one launch");
-    if (att_tile_fits(a)) return att_tile_launch(a, s->batch, st);
+    if (att_tile_fits(a) && !att_rows_faster(a, s->batch)) return att_tile_launch(a, s->batch, st);
     hipLaunchKernelGGL(att_exact, dim3((unsigned)rows), dim3(ATT_THREADS), 0, st, a);
     QBK_HIP(hipGetLastError());
     return QBK_OK;
@@ -579,7 +599,7 @@ int attention_exact_cache(const float *q, const float *kc, const float *vc, size
     if (rows == 0 || H == 0 || Hk == 0 || H % Hk != 0 || hd == 0 || hd > ATT_MAXD)
         return fail(QBK_ERR_VALIDATION, "exact cache attention: bad shape");
     AttArgs a{q, kc, vc, out, H, Hk, 1, rows, hd, hd, 0, 1.0f / sqrtf((float)hd), Hk * hd, hd, Hk * hd, hd};
-    if (att_tile_fits(a)) return att_tile_launch(a, 1, st);
+    if (att_tile_fits(a) && !att_rows_faster(a, 1)) return att_tile_launch(a, 1, st);
     hipLaunchKernelGGL(att_exact, dim3((unsigned)H), dim3(ATT_THREADS), 0, st, a);
     QBK_HIP(hipGetLastError());
     return QBK_OK;

@@ -142,3 +142,22 @@ def test_query_tiles_a_workgroup(ctx, b, h, hk, sq, skv, d, dv):
     for causal in (False, True):
         want, bound = reference(q, k, v, causal)
         assert np.all(np.abs(run(ctx, q, k, v, causal) - want) <= bound)
+
+
+@pytest.mark.parametrize("b,h,hk,sq,skv,d,dv", [
+    (48, 16, 4, 1, 32, 64, 64), (48, 16, 4, 1, 48, 64, 64), (48, 16, 4, 2, 16, 64, 48),   # a row a workgroup, tiles, a row
+    (48, 16, 4, 1, 48, 128, 128), (48, 16, 4, 1, 64, 128, 128), (48, 16, 4, 4, 1, 16, 128),  # a row, tiles, a row
+    (20, 16, 4, 1, 8, 64, 64), (20, 16, 4, 1, 9, 64, 64), (16, 16, 4, 4, 8, 16, 16), (16, 16, 4, 4, 9, 16, 16),
+])
+def test_few_queries_over_few_keys(ctx, b, h, hk, sq, skv, d, dv):
+    """Either side of the line between the row kernel and the tiles."""
+    rng = np.random.default_rng(b + sq + skv + d)
+    q = rng.standard_normal((b, h, sq, d)).astype(np.float32)
+    k = rng.standard_normal((b, hk, skv, d)).astype(np.float32)
+    v = rng.standard_normal((b, hk, skv, dv)).astype(np.float32)
+    for causal in (False, True):
+        want, bound = reference(q, k, v, causal)
+        got = run(ctx, q, k, v, causal)
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        ok = ~np.isnan(want)
+        assert np.all(np.abs(got - want)[ok] <= bound[ok])
