@@ -51,27 +51,27 @@ static unsigned trunk_embed_split(size_t d) {
 // 1 / sqrt(ms + eps), out = bf16(b * inv * w) held as f32.
 // F32: norm_apply at fp32 serving (no bf16 roundings of the operand and
 // the output).
-template <bool F32>
+// PER > 0: rows of up to TRUNK_THREADS * PER elements, read once with every
+// load issued before the first sum; 0: any row, read twice.  The sums run in
+// the same order either way.  A kernel a width, straight-line (loads past the
+// row repeat its first element): with the widest one's registers for every row
+// there were too few waves of many rows.  bf16, us (each row read twice, a load
+// at a time; one kernel of 32 a thread; these): one row of 4096 8.1, 6.4, 3.9;
+// 2048 rows of 64 3.9, 7.6, 3.9, of 4096 20.1, 17.7, 12.2, of 9000 43, 67, 43.
+template <bool F32, int PER>
 __global__ void __launch_bounds__(TRUNK_THREADS) trunk_rms_norm(const float *x, size_t d, const float *w,
                                                                float eps, float *out) {
     __shared__ float red[TRUNK_THREADS / 64];
     const float *xr = x + (size_t)blockIdx.x * d;
     float *orow = out + (size_t)blockIdx.x * d;
-    // Rows of up to TRUNK_THREADS * PER elements: every load issued before
-    // the first sum and the row read once (one at a time, one row of 4096
-    // took 11 us); the sums run in the same order either way.
-    constexpr int PER = 32;
-    const bool held = d <= (size_t)TRUNK_THREADS * PER;
-    float xv[PER], wv[PER];
+    float xv[PER ? PER : 1], wv[PER ? PER : 1];
     float ss = 0.0f;
-    if (held) {
+    if constexpr (PER > 0) {
 #pragma unroll
         for (int k = 0; k < PER; k++) {
             const size_t i = threadIdx.x + (size_t)k * TRUNK_THREADS, c = i < d ? i : 0;
-            if ((size_t)k * TRUNK_THREADS < d) {
-                xv[k] = xr[c];
-                wv[k] = w[c];
-            }
+            xv[k] = xr[c];
+            wv[k] = w[c];
         }
 #pragma unroll
         for (int k = 0; k < PER; k++) {
@@ -95,18 +95,28 @@ __global__ void __launch_bounds__(TRUNK_THREADS) trunk_rms_norm(const float *x, 
 #pragma unroll
     for (int i = 0; i < TRUNK_THREADS / 64; i++) tot += red[i];
     const float inv = 1.0f / sqrtf(tot / (float)d + eps);
-    if (held) {
+    if constexpr (PER > 0) {
 #pragma unroll
         for (int k = 0; k < PER; k++) {
             const size_t i = threadIdx.x + (size_t)k * TRUNK_THREADS;
             if (i < d) orow[i] = F32 ? xv[k] * inv * wv[k] : bf16_to_f32(f32_to_bf16(xv[k] * inv * wv[k]));
         }
-        return;
+    } else {
+        for (size_t i = threadIdx.x; i < d; i += TRUNK_THREADS) {
+            const float b = F32 ? xr[i] : bf16_to_f32(f32_to_bf16(xr[i]));
+            orow[i] = F32 ? b * inv * w[i] : bf16_to_f32(f32_to_bf16(b * inv * w[i]));
+        }
     }
-    for (size_t i = threadIdx.x; i < d; i += TRUNK_THREADS) {
-        const float b = F32 ? xr[i] : bf16_to_f32(f32_to_bf16(xr[i]));
-        orow[i] = F32 ? b * inv * w[i] : bf16_to_f32(f32_to_bf16(b * inv * w[i]));
-    }
+}
+
+template <bool F32>
+static void trunk_rms_norm_launch(const float *x, size_t rows, size_t d, const float *w, float eps, float *out,
+                                  hipStream_t s) {
+    const size_t per = div_ceil(d, TRUNK_THREADS);
+    void (*k)(const float *, size_t, const float *, float, float *) =
+        per <= 2 ? trunk_rms_norm<F32, 2> : per <= 8 ? trunk_rms_norm<F32, 8> : per <= 16 ? trunk_rms_norm<F32, 16>
+        : per <= 32 ? trunk_rms_norm<F32, 32> : trunk_rms_norm<F32, 0>;
+    hipLaunchKernelGGL(k, dim3((unsigned)rows), dim3(TRUNK_THREADS), 0, s, x, d, w, eps, out);
 }
 
 // sampler.rs:4-15 greedy: the first index holding the largest value, a NaN
@@ -238,8 +248,7 @@ int qbk_rms_norm_dev(qbk_ctx *ctx, const float *x, size_t rows, size_t d, const 
     if (!x || !w || !out) return fail(QBK_ERR_VALIDATION, "null argument");
     if (rows == 0 || d == 0) return QBK_OK;
     if ((rc = bind(ctx))) return rc;
-    hipLaunchKernelGGL(trunk_rms_norm<false>, dim3((unsigned)rows), dim3(TRUNK_THREADS), 0, (hipStream_t)stream, x, d,
-                       w, (float)eps, out);
+    trunk_rms_norm_launch<false>(x, rows, d, w, (float)eps, out, (hipStream_t)stream);
     QBK_HIP(hipGetLastError());
     return QBK_OK;
 }
@@ -250,8 +259,7 @@ int qbk_rms_norm_f32_dev(qbk_ctx *ctx, const float *x, size_t rows, size_t d, co
     if (!x || !w || !out) return fail(QBK_ERR_VALIDATION, "null argument");
     if (rows == 0 || d == 0) return QBK_OK;
     if ((rc = bind(ctx))) return rc;
-    hipLaunchKernelGGL(trunk_rms_norm<true>, dim3((unsigned)rows), dim3(TRUNK_THREADS), 0, (hipStream_t)stream, x, d,
-                       w, (float)eps, out);
+    trunk_rms_norm_launch<true>(x, rows, d, w, (float)eps, out, (hipStream_t)stream);
     QBK_HIP(hipGetLastError());
     return QBK_OK;
 }

@@ -50,3 +50,9 @@ def test_rms_norm_rows(ctx, rows, d, serving):
     want = b * torch.rsqrt((b * b).mean(-1, keepdim=True) + 1e-5) * w.double()
     tol = (d + 8) * 2.0 ** -24 + (2.0 ** -8 if serving == "bf16" else 0.0)
     assert bool(((out.double() - want).abs() <= tol * want.abs() + 1e-30).all())
+
+
+@pytest.mark.parametrize("serving", ["bf16", "fp32"])
+@pytest.mark.parametrize("rows,d", [(3, 511), (2, 512), (2, 513), (70, 2048), (2, 2049), (2, 4095), (2, 4097)])
+def test_rms_norm_rows_at_the_kernels_widths(ctx, rows, d, serving):
+    test_rms_norm_rows(ctx, rows, d, serving)
