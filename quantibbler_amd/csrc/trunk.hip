@@ -39,9 +39,12 @@ __global__ void __launch_bounds__(TRUNK_THREADS) trunk_embed_ids(const float *ta
     trunk_embed_row(table, vocab, d, ids.id[blockIdx.x], out + (size_t)blockIdx.x * d);
 }
 
-// Workgroups a row: the row's loads in flight over more CUs than one.
-static unsigned trunk_embed_split(size_t d) {
-    const size_t n = div_ceil(d, 4 * TRUNK_THREADS);
+// Workgroups a row: the row's loads in flight over more CUs than one.  Past
+// 1280 rows one each fills the chip, and more only pass over it in rounds (us,
+// one and split: 1025 rows of 4096 7.7, 6.3, of 9000 15.5, 13.6; 2048 of 4096
+// 11.3, 11.7; 4096 of 9000 70, 80).
+static unsigned trunk_embed_split(size_t rows, size_t d) {
+    const size_t n = rows > 1280 ? 1 : div_ceil(d, 4 * TRUNK_THREADS);
     return (unsigned)(n < 16 ? n : 16);
 }
 
@@ -216,13 +219,13 @@ int qbk_embed(qbk_ctx *ctx, const float *table, size_t vocab, size_t d_model, co
             const size_t c = n - i0 < TRUNK_ARG_IDS ? n - i0 : TRUNK_ARG_IDS;
             TrunkIds a;
             memcpy(a.id, tokens_host + i0, c * 4);
-            hipLaunchKernelGGL(trunk_embed_ids, dim3((unsigned)c, trunk_embed_split(d_model)), dim3(TRUNK_THREADS), 0, s,
+            hipLaunchKernelGGL(trunk_embed_ids, dim3((unsigned)c, trunk_embed_split(c, d_model)), dim3(TRUNK_THREADS), 0, s,
                                table, vocab, d_model, a, out + i0 * d_model);
         }
     } else {
         if ((rc = ids.alloc(n * 4))) return rc;
         QBK_HIP(hipMemcpy(ids.p, tokens_host, n * 4, hipMemcpyHostToDevice));
-        hipLaunchKernelGGL(trunk_embed, dim3((unsigned)n, trunk_embed_split(d_model)), dim3(TRUNK_THREADS), 0, s, table,
+        hipLaunchKernelGGL(trunk_embed, dim3((unsigned)n, trunk_embed_split(n, d_model)), dim3(TRUNK_THREADS), 0, s, table,
                            vocab, d_model, (const int32_t *)ids.p, out);
     }
     QBK_HIP(hipGetLastError());
@@ -236,7 +239,7 @@ int qbk_embed_dev(qbk_ctx *ctx, const float *table, size_t vocab, size_t d_model
     if (!table || !tokens || !out) return fail(QBK_ERR_VALIDATION, "null argument");
     if (n == 0 || d_model == 0) return QBK_OK;
     if ((rc = bind(ctx))) return rc;
-    hipLaunchKernelGGL(trunk_embed, dim3((unsigned)n, trunk_embed_split(d_model)), dim3(TRUNK_THREADS), 0,
+    hipLaunchKernelGGL(trunk_embed, dim3((unsigned)n, trunk_embed_split(n, d_model)), dim3(TRUNK_THREADS), 0,
                        (hipStream_t)stream, table, vocab, d_model, tokens, out);
     QBK_HIP(hipGetLastError());
     return QBK_OK;

@@ -56,3 +56,9 @@ def test_rms_norm_rows(ctx, rows, d, serving):
 @pytest.mark.parametrize("rows,d", [(3, 511), (2, 512), (2, 513), (70, 2048), (2, 2049), (2, 4095), (2, 4097)])
 def test_rms_norm_rows_at_the_kernels_widths(ctx, rows, d, serving):
     test_rms_norm_rows(ctx, rows, d, serving)
+
+
+@pytest.mark.parametrize("n,d", [(1280, 1030), (1281, 1030), (3000, 2049)])
+def test_embed_many_rows(ctx, n, d):
+    """Either side of where a row stops being split over workgroups."""
+    test_embed_rows(ctx, n, d)
