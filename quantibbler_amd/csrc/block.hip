@@ -1292,7 +1292,7 @@ int qbk_block_prefill_seq_dev(qbk_ctx *ctx, qbk_block *B, size_t seq, float *h, 
     blkp_norm_launch(n, oo, h, h1, B->w_post, B->eps, x, d, 1, s);
     QBK_HIP(hipGetLastError());
     if ((rc = blkp_proj(B->lay[4], n, x, false, g, ws, s))) return rc;
-    if (n > Q4_MAXB && q4g_use(B->lay[5], n) && q4g_use(B->down, n) && B->ffn % 4 == 0) {
+    if (n > Q4_MAXB && q4g_use(B->lay[5], n) && q4g_use(B->down, n) && B->ffn % 4 == 0 && (uintptr_t)w % 8 == 0) {
         // the up projection's epilogue forms SwiGLU and from it the down
         // projection's z in bf16 (read at s2 = 1): u never goes to memory;
         // h = down + h1, the residual added in the GEMM's epilogue
