@@ -717,8 +717,7 @@ static BlkpPlan blkp_plan(const qbk_block *B, const qbk_factor *const L[7], size
     p.o_oo = take(n * d * 4);
     p.o_h1 = take(n * d * 4);
     p.o_g = take(n * B->ffn * 4);
-    p.o_u = take(n * B->ffn * 4);
-    p.o_z = take(n * B->ffn * 2);
+    p.o_u = p.o_z = take(n * B->ffn * 4);  // the up projection's f32 rows, or the down projection's z without them
     size_t g = 0;
     for (int i = 0; i < 7; i++) {
         const size_t w = blkp_proj_ws(L[i], n);

@@ -84,3 +84,17 @@ def test_swiglu_in_the_epilogue_is_the_separate_pass(orc, n, ffn, r):
         outs.append(prefill(block, h))
         block.close()
     assert np.isfinite(outs[0]).all() and outs[0].tobytes() == outs[1].tobytes()
+
+
+def test_prompt_workspace_holds_two_ffn_rows(orc):
+    """The gate projection's f32 rows, and one region for the up projection's or
+    the z that its epilogue leaves: 8 bytes for each further ffn row and token."""
+    from quantibbler_amd import GpuContext
+
+    ctx, n = GpuContext(0), 300
+    need = []
+    for ffn in (512, 1024):
+        block = make_block(orc, ctx, ffn, 256, ffn, 2, 1, n)
+        need.append(block.prefill_workspace_size(n))
+        block.close()
+    assert need[1] - need[0] == n * 512 * 8
