@@ -143,3 +143,22 @@ def test_exact_face_validation_texts(ctx):
         with pytest.raises(KernelError) as e:
             ctx.attention(shape, q, q, q, False)
         assert str(e.value) == text
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("sq,skv,d,dv", [(5, 1025, 160, 160), (3, 2500, 300, 300), (4, 2100, 20, 36), (1, 1024, 130, 64),
+                                         (2, 3000, 64, 1024), (3, 1100, 1024, 17)])
+def test_exact_face_row_kernel_over_chunks_of_keys(ctx, sq, skv, d, dv, causal):
+    """Shapes that the tiles do not take (dims past 128 or not of 16), over more
+    than the 1024 keys of the row kernel's chunk: its online softmax, its
+    several output channels a thread, the largest dims."""
+    from quantibbler_amd import AttentionShape
+
+    say("exact attention rows", sq, skv, d, dv, causal)
+    rng = np.random.default_rng(sq + skv + d + dv)
+    q = rng.standard_normal((1, 4, sq, d)).astype(np.float32)
+    k = rng.standard_normal((1, 2, skv, d)).astype(np.float32)
+    k[:, :, skv // 2:] *= 1.5                  # the largest scores after the first chunk
+    v = rng.standard_normal((1, 2, skv, dv)).astype(np.float32)
+    got = ctx.attention(AttentionShape(1, 4, 2, sq, skv, d, dv), q, k, v, causal)
+    two_part(got, dense(*(a.astype(np.float64) for a in (q, k, v)), causal), dv)

@@ -86,6 +86,46 @@ def test_swiglu_in_the_epilogue_is_the_separate_pass(orc, n, ffn, r):
     assert np.isfinite(outs[0]).all() and outs[0].tobytes() == outs[1].tobytes()
 
 
+@pytest.mark.parametrize("H,Hk,qk_norm", [(2, 1, True), (3, 1, False), (16, 8, True), (13, 1, True)])
+def test_rope_in_16_byte_pieces_keeps_the_sums(orc, H, Hk, qk_norm):
+    """A prompt's cache rows against those that a batched decode step writes at
+    the same positions, one a sequence: its RoPE runs a wave a head, with the
+    tree of sums that the prompt's sixteen lanes keep."""
+    from quantibbler_amd import GpuContext
+
+    n, d = 8, 256
+    print("prompt rope bits", H, Hk, qk_norm, flush=True)
+    ctx = GpuContext(0)
+    block = make_block(orc, ctx, 10 * H + Hk, d, 256, H, Hk, n, n_seqs=n, qk_norm=qk_norm)
+    h = np.random.default_rng(H).standard_normal((n, d)).astype(np.float32)
+    width = Hk * 128
+
+    def caches():
+        out = []
+        for ptr in block.cache_ptrs():
+            sto = torch._C._construct_storage_from_data_pointer(ptr, torch.device("cuda", 0), n * n * width * 4)
+            out.append(torch.empty(0, dtype=torch.float32, device="cuda")
+                       .set_(sto, 0, (n, n, width), (n * width, width, 1)))
+        return out
+
+    for c in caches():
+        c.zero_()
+    prefill(block, h)
+    want = [c[0].cpu().numpy() for c in caches()]  # sequence 0's rows 0 .. n - 1
+    for c in caches():
+        c.zero_()
+    block.set_filled(list(range(n)))
+    rows = torch.from_numpy(h).cuda()
+    need = block.decode_batch_workspace_size(n)
+    block.decode_batch_dev(rows, list(range(n)), torch.empty(need, dtype=torch.uint8, device="cuda"), need,
+                           torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    for c, w in zip(caches(), want):
+        got = np.stack([c[i, i].cpu().numpy() for i in range(n)])
+        assert np.abs(w).sum(axis=1).min() > 0 and got.tobytes() == w.tobytes()
+    block.close()
+
+
 def test_prompt_workspace_holds_two_ffn_rows(orc):
     """The gate projection's f32 rows, and one region for the up projection's or
     the z that its epilogue leaves: 8 bytes for each further ffn row and token."""
