@@ -43,6 +43,7 @@
 // (2048 tokens of 14336: 235 MB read, 45 us) goes; the exps add about 25 us
 // to the launch.
 #include <mutex>
+#include <type_traits>
 
 #include "factor_internal.h"
 #include "q4_operand.h"
@@ -73,10 +74,15 @@ struct Q4GArgs {
     uint16_t *t_out;                // t bf16 [N][r_p] as well (zero past r), or null
     uint32_t r_p;
     const float *resid;             // f32 [N][dout] added to an f32 y (the block's residual), or null
-    // bf16 y only, or null: y is then z = bf16(zs2 hid), hid = gate y / (1 +
-    // exp(-gate)) -- the block's SwiGLU of this layer (up) and the gate
-    // projection's f32 rows, as the down projection's z
-    const float *gate, *zs2;        // f32 [N][dout], [dout]
+};
+
+// Of the kernels with a gate (bf16 y only): y is z = bf16(zs2 hid), hid = gate
+// y / (1 + exp(-gate)) -- the block's SwiGLU of this layer (up) and the gate
+// projection's f32 rows, as the down projection's z.  (A type of their own:
+// with these fields in Q4GArgs the plain kernels' argument loads and branches
+// came out otherwise.)
+struct Q4GGateArgs : Q4GArgs {
+    const float *gate, *zs2;  // f32 [N][dout], [dout]
 };
 
 __device__ __forceinline__ i32x8_t q4g_signs(uint32_t w, uint32_t c7) {
@@ -308,11 +314,12 @@ __device__ __forceinline__ uint32_t q4g_pair_u(uint32_t v) {
 // so waiting for them drains the ring, and as a branch of the plain kernels
 // they took the counts of those down with them (4096 x 4096 of rank 1024, 2048
 // tokens: 33.3 -> 33.7 us with bf16 y, 34.9 -> 36.5 with f32).
-template <bool VECY, bool GATE>
-__device__ __forceinline__ void q4g_epilogue2(const f32x4_t acc[4], const Q4GArgs &a, size_t g, const float *sb,
+template <bool VECY, class Args>
+__device__ __forceinline__ void q4g_epilogue2(const f32x4_t acc[4], const Args &a, size_t g, const float *sb,
                                               size_t n0, int lane, bool ybf16) {
     const int col = lane & 15, G = lane >> 4, odd = col & 1;
     const size_t n = n0 + (col >> 1);
+    constexpr bool GATE = std::is_same<Args, Q4GGateArgs>::value;
     float2 gv[4], zv[4];
     if constexpr (GATE) {  // the group's gate values and scales, all in flight
         const size_t nc = n < a.N ? n : a.N - 1;
@@ -390,8 +397,8 @@ __device__ __forceinline__ void q4g_prio(uint32_t level) {
 // NG1: stage-1 row groups a wave accumulates (1: r_p <= 1024, 2: r_p <=
 // 2048).  Stage 1's unit: one slice of the wave's NG1 row groups (their B
 // fragment read once); stage 2's unit: one slice of a pair of row groups.
-template <bool XF32, bool YBF16, int NG1, bool VECY, bool GATE = false>
-__global__ void __launch_bounds__(64 * Q4G_WAVES) q4g_kernel(Q4GArgs a) {
+template <bool XF32, bool YBF16, int NG1, bool VECY, class Args = Q4GArgs>
+__global__ void __launch_bounds__(64 * Q4G_WAVES) q4g_kernel(Args a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t q4g_lds[];
     uint8_t *xbuf = q4g_lds;                             // [2][Q4G_CH slices]
     uint8_t *tbuf = q4g_lds + 2 * Q4G_CH * Q4G_SLICE;    // [ns2 slices]
@@ -563,8 +570,8 @@ __global__ void __launch_bounds__(64 * Q4G_WAVES) q4g_kernel(Q4GArgs a) {
         __builtin_amdgcn_wave_barrier();
         Q4G_SCALES2(p + 1 < np2 ? p + 1 : p)
         const size_t g0 = (size_t)wave + Q4G_WAVES * (2 * p);
-        q4g_epilogue2<VECY, GATE>(acc2[0], a, g0, sb, n0, lane, YBF16);
-        if (two) q4g_epilogue2<VECY, GATE>(acc2[1], a, g0 + Q4G_WAVES, sb + 128, n0, lane, YBF16);
+        q4g_epilogue2<VECY>(acc2[0], a, g0, sb, n0, lane, YBF16);
+        if (two) q4g_epilogue2<VECY>(acc2[1], a, g0 + Q4G_WAVES, sb + 128, n0, lane, YBF16);
         __builtin_amdgcn_wave_barrier();
     }
 #undef Q4G_ISSUE2
@@ -584,8 +591,8 @@ static const void *const q4g_kernels[18] = {
     Q4G_K(false, true, 2, false),  Q4G_K(false, true, 2, true),  Q4G_K(true, false, 1, false),
     Q4G_K(true, false, 1, true),   Q4G_K(true, false, 2, false), Q4G_K(true, false, 2, true),
     Q4G_K(true, true, 1, false),   Q4G_K(true, true, 1, true),   Q4G_K(true, true, 2, false),
-    Q4G_K(true, true, 2, true),    (const void *)q4g_kernel<false, true, 1, true, true>,
-    (const void *)q4g_kernel<false, true, 2, true, true>};
+    Q4G_K(true, true, 2, true),    (const void *)q4g_kernel<false, true, 1, true, Q4GGateArgs>,
+    (const void *)q4g_kernel<false, true, 2, true, Q4GGateArgs>};
 #undef Q4G_K
 
 // x chunks, stage 2's operand, each wave's s1 / bias staging (1 KiB)
@@ -640,7 +647,7 @@ int q4g_run(const qbk_factor *L, const void *x, bool xf32, size_t N, void *y, bo
             done |= 1ull << dev;
         }
     }
-    Q4GArgs a{};
+    Q4GGateArgs a{};
     a.bits1 = L->vt_q4;
     a.bits2 = L->u_q4;
     a.s2 = s2 ? s2 : L->s2;
@@ -668,7 +675,7 @@ int q4g_run(const qbk_factor *L, const void *x, bool xf32, size_t N, void *y, bo
     // one row group a wave in stage 1 up to 16 groups (r_p <= 1024), two up to 32
     const bool two = a.n_rg1 > Q4G_WAVES;
     const void *k = q4g_kernels[gate ? 16 + two : (xf32 ? 8 : 0) | (ybf16 ? 4 : 0) | (two ? 2 : 0) | (a.vec_y ? 1 : 0)];
-    void *args[] = {&a};
+    void *args[] = {static_cast<Q4GArgs *>(&a)};  // the plain kernels read the base alone
     QBK_HIP(hipLaunchKernel(k, grid, block, args, lds, s));
     QBK_HIP(hipGetLastError());
     return QBK_OK;
