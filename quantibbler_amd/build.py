@@ -11,7 +11,7 @@ quantibbler_amd/libqbk.so, which the ctypes binding loads.  Flags:
                                 no packed FP32 VALU ops (the host pass warns
                                 that it does not know the feature; harmless)
 Per source (EXTRA):
-  decode.hip: -mllvm -amdgpu-mfma-vgpr-form=1
+  decode.hip, gemm.hip, serve64.hip: -mllvm -amdgpu-mfma-vgpr-form=1
                                 MFMA accumulators in VGPRs: the GEMV's
                                 accumulators cross branches (partial load
                                 steps), and in AGPRs every crossing copied

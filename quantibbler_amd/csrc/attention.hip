@@ -164,9 +164,10 @@ __global__ void __launch_bounds__(ATT_THREADS) att_exact(AttArgs a) {
 // What bounds it: the operands' way into registers (a 1 KB wave load takes
 // about 40 cycles of the CU's, which the f32 MFMAs, 32 cycles each for 2048
 // FLOP, only half cover: without the loads 2 x 777 queries run at 154 TFLOP/s,
-// the card's f32 rate).  Measured: 16 / 8 heads, 777 queries over 1300 keys,
-// d 128, causal: 5.34 ms with a row a workgroup, 0.11 ms here; one query of
-// 32 / 8 heads over 700 keys 130 -> 28 us.
+// the card's f32 rate).  Measured, a row a workgroup -> here: 16 / 8 heads, 777
+// queries over 1300 keys, d 128, causal 5.33 -> 0.103 ms; one query of 32 / 8
+// heads over 700 keys 128 -> 28 us (over a block's cache, whose rows hold all
+// heads, 227 -> 29 under the profiler).
 #define ATT_TILE_K 32  // keys a wave takes at a time
 #define ATT_WAVES 8    // waves a workgroup, the key tiles among them
 

@@ -432,7 +432,7 @@ __global__ void __launch_bounds__(NT) blkp_norm(const float *__restrict__ a, con
 // its loads issued at once.  The bf16 row passes through LDS, from which
 // thread t sums channels t, t + 256, .. in turn, as blkp_norm<256>'s does:
 // every value is that kernel's, bit for bit.  HBM-bound: 2048 rows of 4096,
-// 4-byte accesses -> these, 21 -> 11 us without a residual (50 MB), 41 -> 20 us
+// 4-byte accesses -> these, 21 -> 10 us without a residual (50 MB), 41 -> 19 us
 // with one (117 MB).  (A wave a row, whose lanes hold such sums whole, takes
 // the same at 2048 rows and 4 us more a launch at 65 to 777.)
 // NE: 16-byte pieces a thread, 1024 NE >= d.
@@ -583,7 +583,8 @@ __global__ void __launch_bounds__(256) blkp_qk_rope(const float *q, const float 
     }
 }
 
-// blkp_qk_rope at a head dim of 128 and 16-byte aligned operands: 16 lanes a
+// blkp_qk_rope at a head dim of 128 and 16-byte aligned operands (a prompt's,
+// but for a workspace that is not; that one takes blkp_qk_rope): 16 lanes a
 // head, each four channels of either half in 16-byte loads (the bf16 rows in
 // 8-byte stores), every load issued at once; the v heads are units of their
 // own.  The squares' sum takes blkp_qk_rope's tree -- channel j

@@ -313,7 +313,8 @@ __device__ __forceinline__ uint32_t q4g_pair_u(uint32_t v) {
 // its own for the same reason: its gate loads go out behind the ring's refill,
 // so waiting for them drains the ring, and as a branch of the plain kernels
 // they took the counts of those down with them (4096 x 4096 of rank 1024, 2048
-// tokens: 33.3 -> 33.7 us with bf16 y, 34.9 -> 36.5 with f32).
+// tokens: 33.3 -> 33.7 us with bf16 y, 34.9 -> 36.5 with f32; 14336 x 4096 of
+// rank 1700, 256 tokens 89.4 -> 91.1).
 template <bool VECY, class Args>
 __device__ __forceinline__ void q4g_epilogue2(const f32x4_t acc[4], const Args &a, size_t g, const float *sb,
                                               size_t n0, int lane, bool ybf16) {

@@ -550,9 +550,10 @@ __global__ void __launch_bounds__(REF_ROWS) sage_ref_main(RefArgs a) {
 // update ~1000, the shifts ~500; few waves a SIMD) sets the pace: K^ and its
 // deltas are loaded a block ahead and V^ ahead of the softmax, so that no
 // load is waited for.  Measured (16 / 8 heads, d 128, 1999 tokens, causal,
-// block 64): a query per lane and v_dot4 (sage_ref_main) 10.16 ms a call,
-// this 0.109 ms; block 128 at 1800 tokens, 8 heads, 9.05 -> 0.095 ms; d 64,
-// block 32, not causal, 1900 tokens, 8 heads, 5.18 -> 0.085 ms.
+// block 64): a query per lane and v_dot4 (sage_ref_main) 10.20 ms a call,
+// this 0.115 ms (the kernel 0.104 under the profiler, sage_ref_prep 0.016);
+// 8 / 4 heads, block 128, 1800 tokens, causal, 8.95 -> 0.108 ms; d 64, block
+// 32, not causal, 1900 tokens, 5.20 -> 0.097 ms.
 #define REF_TILE_Q 64  // queries a workgroup
 #define REF_TILE_AHEAD 4  // key blocks whose shifts are formed together (one a wave)
 

@@ -28,8 +28,8 @@ __global__ void __launch_bounds__(TRUNK_THREADS) trunk_embed(const float *table,
     trunk_embed_row(table, vocab, d, tokens[blockIdx.x], out + (size_t)blockIdx.x * d);
 }
 
-// Host ids as a kernel argument: no device buffer, copy or free a call (those
-// cost a decode step's call about 20 us of host and device time).
+// Host ids as a kernel argument: no device buffer, copy or free a call (one row
+// of 4096, the call by itself 29.8 -> 14.4 us).
 #define TRUNK_ARG_IDS 256
 struct TrunkIds {
     int32_t id[TRUNK_ARG_IDS];

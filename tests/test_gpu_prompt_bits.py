@@ -1,7 +1,6 @@
 """GPU: a prompt's faster kernels against the general ones they stand in for,
-bit for bit.  A row stream h that is not 16-byte aligned takes the general
-norm (and the element-wise GEMM store), so the same prompt at an aligned and
-at an unaligned h must leave the same bits."""
+bit for bit: norms and RoPE in 16-byte pieces, SwiGLU in the up projection's
+epilogue."""
 import numpy as np
 import pytest
 
@@ -41,6 +40,8 @@ def prefill(block, h, shift=0):
 
 @pytest.mark.parametrize("n,d", [(65, 4), (70, 252), (66, 256), (256, 260), (300, 1028), (68, 4096), (67, 4100), (65, 8192)])
 def test_norm_in_16_byte_pieces_keeps_the_sums(orc, n, d):
+    """A row stream h that is not 16-byte aligned takes the general norm (and the
+    element-wise GEMM store): the same prompt leaves the same bits."""
     from quantibbler_amd import GpuContext
 
     print("prompt norm bits", n, d, flush=True)
