@@ -998,8 +998,8 @@ static int block_decode_f32(qbk_ctx *ctx, qbk_block *B, float *h, size_t pos, hi
         B->tokens[0] = pos + 1;
     }
     B->filled[0] = pos + 1;
-    float *const oo = B->oout, *const gu[2] = {B->ycat, B->ycat + ffn}, *const out = h;
-    if ((rc = factor_f64_run(B->lay + 3, 1, B->attn, &oo, B->f64s, s))) return rc;
+    float *const gu[2] = {B->ycat, B->ycat + ffn}, *const out = h;
+    if ((rc = factor_f64_run(B->lay[3], B->attn, B->oout, B->f64s, s))) return rc;
     hipLaunchKernelGGL(blkd_norm_z, dim3(1), dim3(BLKD_NORM_THREADS), 0, s, (const float *)B->oout, (const float *)h,
                        B->h1, (const float *)B->w_post, B->eps, feeds(B->lay + 4, 2), 2, d);
     QBK_HIP(hipGetLastError());

@@ -430,8 +430,9 @@ int qbk_factor_apply(qbk_ctx *ctx, const qbk_factor *L, int serving, const float
             return rc;
         QBK_HIP(hipMemcpyAsync(dx.p, x, batch * L->din * 4, hipMemcpyHostToDevice, cs.s));
         for (size_t bb = 0; bb < batch; bb++) {
-            float *yb = (float *)dy.p + bb * L->dout;
-            if ((rc = factor_f64_run(&L, 1, (const float *)dx.p + bb * L->din, &yb, (double *)dsc.p, cs.s))) return rc;
+            if ((rc = factor_f64_run(L, (const float *)dx.p + bb * L->din, (float *)dy.p + bb * L->dout, (double *)dsc.p,
+                                     cs.s)))
+                return rc;
         }
         QBK_HIP(hipMemcpyAsync(y, dy.p, batch * L->dout * 4, hipMemcpyDeviceToHost, cs.s));
         QBK_HIP(hipStreamSynchronize(cs.s));

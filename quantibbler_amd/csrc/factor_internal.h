@@ -163,9 +163,9 @@ int g32_run(const qbk_factor *L, const void *x, bool xf32, size_t N, void *y, bo
 // (a group sharing an input, or one), in two launches after z.  The layers'
 // signs must be formed (factor_f64_ready, once a layer).  scratch holds
 // factor_f64_scratch doubles: per layer z then t, each in f64_pos order and
-// zero past its valid length to a multiple of 128.  factor_f64_run forms z
-// from x; factor_f64_staged runs from a z that a caller's kernel has written
-// at factor_f64_z (resid, or null, is added to every y).
+// zero past its valid length to a multiple of 128.  factor_f64_run forms one
+// layer's z from x; factor_f64_staged runs from the z that a caller's kernel has
+// written at factor_f64_z (resid, or null, is added to every y).
 #define F64_MAXL 3
 __host__ __device__ inline uint32_t f64_pos(uint32_t k) {  // pairs k, k + 4 side by side: a 16-byte load a lane group
     return (k & ~7u) | ((k & 3u) << 1) | ((k >> 2) & 1u);
@@ -175,6 +175,6 @@ size_t factor_f64_scratch(const qbk_factor *const *L, int n);
 double *factor_f64_z(const qbk_factor *const *L, int i, double *scratch);
 int factor_f64_staged(const qbk_factor *const *L, int n, float *const *y, const float *resid, double *scratch,
                       hipStream_t s);
-int factor_f64_run(const qbk_factor *const *L, int n, const float *x, float *const *y, double *scratch, hipStream_t s);
+int factor_f64_run(const qbk_factor *L, const float *x, float *y, double *scratch, hipStream_t s);
 
 }  // namespace qbk

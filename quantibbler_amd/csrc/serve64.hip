@@ -180,16 +180,11 @@ __global__ void __launch_bounds__(64) f64_stage(F64Args a) {
     }
 }
 
-// z = f64(s2 * x), an f32 product widened, zero past din (grid y: the layer)
-struct F64In {
-    const float *s2[F64_MAXL];
-    double *z[F64_MAXL];
-    uint32_t din[F64_MAXL];
-};
-__global__ void f64_in(const float *x, F64In a) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, l = blockIdx.y, din = a.din[l];
+// z = f64(s2 * x), an f32 product widened, zero past din
+__global__ void f64_in(const float *x, const float *s2, double *z, uint32_t din) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= ((din + 127) & ~127u)) return;
-    a.z[l][f64_pos(i)] = i < din ? (double)(a.s2[l][i] * x[i]) : 0.0;
+    z[f64_pos(i)] = i < din ? (double)(s2[i] * x[i]) : 0.0;
 }
 
 int factor_f64_ready(const qbk_factor *L, hipStream_t s) {
@@ -251,18 +246,11 @@ int factor_f64_staged(const qbk_factor *const *L, int n, float *const *y, const 
     return QBK_OK;
 }
 
-int factor_f64_run(const qbk_factor *const *L, int n, const float *x, float *const *y, double *scratch, hipStream_t s) {
-    F64In in{};
-    size_t most = 0;
-    for (int i = 0; i < n; i++) {
-        in.s2[i] = L[i]->s2;
-        in.z[i] = factor_f64_z(L, i, scratch);
-        in.din[i] = (uint32_t)L[i]->din;
-        most = L[i]->din_q > most ? L[i]->din_q : most;
-    }
-    hipLaunchKernelGGL(f64_in, dim3((unsigned)div_ceil(most, 256), (unsigned)n), dim3(256), 0, s, x, in);
+int factor_f64_run(const qbk_factor *L, const float *x, float *y, double *scratch, hipStream_t s) {
+    hipLaunchKernelGGL(f64_in, dim3((unsigned)div_ceil(L->din_q, 256)), dim3(256), 0, s, x, (const float *)L->s2,
+                       factor_f64_z(&L, 0, scratch), (uint32_t)L->din);
     QBK_HIP(hipGetLastError());
-    return factor_f64_staged(L, n, y, nullptr, scratch, s);
+    return factor_f64_staged(&L, 1, &y, nullptr, scratch, s);
 }
 
 }  // namespace qbk
