@@ -492,9 +492,9 @@ static bool att_tile_fits(const AttArgs &a) {
 // 7.5 us), while the rows of att_exact share one and cost by their keys.
 // Measured over 3150 shapes (heads 32 to 16384, queries 1 to 16, keys 1 to
 // 128, d 16 to 128), row kernel against tiles, us: 4096 heads of d 64, one
-// query, 1 key 18, 66; 32 keys 48, 67; 48 keys and more the tiles; two queries,
-// 16 keys 58, 71; four queries, 8 keys 82, 72; d 128, one query, 32 keys 68,
-// 124; 64 keys 162, 125.  Up to 256 heads every workgroup of att_tile has a CU
+// query, 1 key 18, 66; 32 keys 48, 68; 48 keys 82, 75; two queries, 16 keys 63,
+// 72; four queries, 8 keys 93, 69; d 128, one query, 32 keys 68, 124; 48 keys
+// 125, 140; 64 keys 162, 136.  Up to 256 heads every workgroup of att_tile has a CU
 // at once and only rows of 16 channels or fewer are better off by themselves.
 // (Heads: batches times heads.)
 static bool att_rows_faster(const AttArgs &a, size_t B) {
@@ -515,9 +515,9 @@ static int att_tile_launch(AttArgs a, size_t B, hipStream_t st) {
     // 44 each.
     // Tiles that hold no query leave their waves idle, so no more of them than
     // there are queries for where the keys need the waves: 4096 single queries
-    // (us for 1 and 4 tiles) over 32 keys of d 64 67, 72; 64 keys 67, 82; 128
-    // keys 74, 121; 16 queries of 1024 heads over 32 keys 26, 22 (the merge of
-    // eight waves' outputs); 64 keys 26, 27.
+    // (us for 1 and 4 tiles) over 32 keys of d 64 68, 72; 64 keys 72, 91; 128
+    // keys 82, 137; 16 queries of 1024 heads over 32 keys 25, 21 (the merge of
+    // eight waves' outputs); 64 keys 27, 28.
     int qw = div_ceil(a.Sq, 64) * B * a.H >= 400 ? 4 : div_ceil(a.Sq, 32) * B * a.H >= 150 ? 2 : 1;
     if (a.Skv >= 32 + 6 * a.Sq)
         while (qw > 1 && 8 * (size_t)qw >= a.Sq) qw /= 2;
